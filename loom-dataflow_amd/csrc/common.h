@@ -171,11 +171,15 @@ static inline int loom_ok(char* err, size_t errlen) {
   return LOOM_OK;
 }
 
-static inline int loom_check_launch(char* err, size_t errlen, const char* what) {
-  hipError_t e = hipGetLastError();
+// The status of a launch whose error has been taken already.
+static inline int loom_launched(hipError_t e, char* err, size_t errlen, const char* what) {
   if (e != hipSuccess)
     return loom_fail(err, errlen, LOOM_EHIP, "%s: launch failed: %s", what, hipGetErrorString(e));
   return loom_ok(err, errlen);
+}
+
+static inline int loom_check_launch(char* err, size_t errlen, const char* what) {
+  return loom_launched(hipGetLastError(), err, errlen, what);
 }
 
 static inline int64_t cdiv64(int64_t a, int64_t b) { return (a + b - 1) / b; }

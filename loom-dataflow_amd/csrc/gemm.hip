@@ -16,8 +16,11 @@
 //                        software-pipelined LDS-DMA stages with the MFMA
 //                        fragments of the next stage read during this one.
 //   gemm_dma_kernel      256x256 tiles, LDS-DMA stages, K a multiple of 32.
-//   gemm_bf16_kernel     any shape: register-staged 64-deep tiles (half of the
-//                        threads copy A rows, the other half copy 8x8 blocks of
+//   gemm_ragged_kernel<T> rows off 16-byte boundaries (K or N not a multiple of
+//                        8): 16-byte register loads at any element, the
+//                        pipelined kernels' LDS layouts.
+//   gemm_bf16_kernel     any other shape: register-staged 64-deep tiles (half of
+//                        the threads copy A rows, the other half copy 8x8 blocks of
 //                        B, transpose them in registers and store B^T), LDS rows
 //                        of 128 bytes XOR-swizzled by (row & 7).
 // All compute C^T tiles with v_mfma_f32_16x16x32_bf16 (B^T as the row
@@ -1028,6 +1031,306 @@ bool launch_persist(const GemmParams& p, bool aligned, bool out_f32, hipStream_t
   return true;
 }
 
+// ---------------------------------------------------------------------------
+// Ragged operands (T x T tile, T = 64 or 128): rows of A, B or C that do not
+// start on 16-byte boundaries (K or N not a multiple of 8, or a tensor based
+// off one), which LDS DMA cannot copy.  Every piece is still one 16-byte
+// access, at whatever 2-byte aligned address it starts: ROCm's driver runs
+// every GPU process in the unaligned access mode (SH_MEM_CONFIG.alignment_mode
+// UNALIGNED), where dword and wider global accesses take any byte address.
+// The pieces go through registers into the pipelined kernels' LDS layouts
+// (A [T][BK], B [BK][T], the same swizzles and transposed reads), R stages in
+// flight per thread (up to 64 VGPRs of loads) over two LDS stages and one
+// barrier per stage.
+//
+// No access leaves the operands.  Rows past M repeat the last one and are
+// never stored.  The last K stage may be partial: a piece of A that would
+// pass the range's end ke is loaded ending there and shifted down, so its
+// elements past ke are zeros; rows of B past ke are zeros too (both, so an
+// infinity or NaN beside the range meets no zero factor).  A piece of B that
+// would pass column N is loaded ending there and shifted down; its columns
+// past N are never stored.  Needs ke >= 8 and N >= 8.
+//
+// Bound: the loads' issue.  A 16-byte load at an odd element costs about four
+// times one on a dword (T 64, 2048^3: 36 us with every row on a dword, 67 us
+// with every row off one), and half of an odd extent's rows start at one; then
+// the step's chain of LDS store, barrier, LDS read and MFMA, which two or three
+// workgroups per CU overlap.  Against the element-load kernel (eight 2-byte
+// loads a piece) that ran these shapes before, M 1003 N 1531 K 2051: 214 ->
+// 26 us (242 TFLOP/s).  Four stages of loads in flight instead of two took the
+// same time and 64 more VGPRs; the odd pieces as an aligned 16-byte load, the
+// next dword and a byte shift: 27 against 35 us on the 64 tile (every row odd,
+// 1024x1536x2048) but 47 against 35 on the 128 tile.
+// ---------------------------------------------------------------------------
+typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));   // 16 bytes at any element
+
+// Elements e .. 7 of v moved to 0 .. 7 - e, zeros behind them (e >= 8: zero).
+LOOM_DEV u32x4_t shift_down(const u32x4_t& v, int e) {
+  uint64_t lo = ((uint64_t)v[1] << 32) | v[0], hi = ((uint64_t)v[3] << 32) | v[2];
+  const int b = 16 * (e & 3);
+  if (e & 4) {
+    lo = hi;
+    hi = 0;
+  }
+  if (b) {
+    lo = (lo >> b) | (hi << (64 - b));
+    hi >>= b;
+  }
+  if (e >= 8) lo = hi = 0;
+  return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
+template <int T, bool OUT_F32, bool H>
+__global__ void __launch_bounds__(256, 2) gemm_ragged_kernel(GemmParams p) {
+  constexpr int BK = T == 64 ? 64 : 32;          // K depth of a stage
+  constexpr int R = 2;                           // stages of loads in flight
+  constexpr int TT = T / 32;                     // 16-wide tiles per wave dimension
+  constexpr int A_BYTES = T * BK * 2, B_BYTES = BK * T * 2, STAGE = A_BYTES + B_BYTES;
+  constexpr int A_ROW = BK * 2, B_ROW = T * 2;
+  constexpr int AP = A_BYTES / 4096, BP = B_BYTES / 4096;   // pieces per thread and stage
+  constexpr int ES = OUT_F32 ? 4 : 2, C_ROW = T * ES;
+  constexpr int SMEM = 2 * STAGE > T * C_ROW ? 2 * STAGE : T * C_ROW;
+  static_assert(R % 2 == 0, "an LDS stage is fixed by the ring slot");
+  __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+  lds_char_t* const lds = (lds_char_t*)smem;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // ---- which tile, which z (XCD-contiguous, grouped by 8 tile rows)
+  const int nblocks = p.tiles_m * p.tiles_n * p.nz;
+  const int bid = xcd_remap(blockIdx.x, nblocks);
+  const int per_z = p.tiles_m * p.tiles_n;
+  const int z = bid / per_z;
+  const int t = bid - z * per_z;
+  constexpr int GM = 8;
+  const int group = t / (GM * p.tiles_n);
+  const int first_m = group * GM;
+  const int gsz = min(p.tiles_m - first_m, GM);
+  const int tin = t - group * GM * p.tiles_n;
+  const int64_t m0 = (int64_t)(first_m + tin % gsz) * T;
+  const int64_t n0 = (int64_t)(tin / gsz) * T;
+
+  const uint16_t* A = p.A;
+  const uint16_t* B = p.B;
+  int64_t kb = 0, ke = p.k_total;
+  if (p.split) {
+    kb = (int64_t)z * p.k_slab;
+    ke = min(p.k_total, kb + p.k_slab);
+  } else {
+    A += (int64_t)z * p.za;
+    B += (int64_t)z * p.zb;
+  }
+  const int nfull = (int)((ke - kb) / BK), rem = (int)((ke - kb) % BK);
+  const int ns = nfull + (rem != 0);
+
+  // ---- per-lane byte offsets of the pieces: against the stage's base, and
+  // against the partial stage's (at*: its base column is 8 before its first,
+  // so the pieces that end at ke stay at or after it)
+  const int64_t kt = kb + (int64_t)nfull * BK;          // first column of the partial stage
+  const int64_t at0 = max<int64_t>(kt - 8, 0);
+  uint32_t aoff[AP], atoff[AP], boff[BP], btoff[BP];
+  int ash[AP], bsh[BP];       // elements to shift down by: partial stage, last columns
+  int brow[BP];
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int e = (wave * AP + i) * 1024 + lane * 16;
+    const int row = e / A_ROW, kc = ((e % A_ROW) / 16) ^ a_swz<BK>(row);
+    const int64_t gm = min<int64_t>(row, p.M - 1 - m0);
+    const int64_t k = kt + kc * 8, kl = min<int64_t>(k, ke - 8);
+    aoff[i] = (uint32_t)(gm * p.lda * 2 + kc * 16);
+    atoff[i] = (uint32_t)(gm * p.lda * 2 + (kl - at0) * 2);
+    ash[i] = (int)(k - kl);
+  }
+#pragma unroll
+  for (int i = 0; i < BP; ++i) {
+    const int e = (wave * BP + i) * 1024 + lane * 16;
+    const int row = e / B_ROW, nc = ((e % B_ROW) / 16) ^ b_swz_t<T>(row);
+    const int64_t n = n0 + nc * 8, nl = min<int64_t>(n, p.N - 8);
+    brow[i] = row;
+    boff[i] = (uint32_t)(row * p.ldb * 2 + (nl - n0 + 8) * 2);   // base column n0 - 8: never negative
+    btoff[i] = (uint32_t)(min<int64_t>(row, ke - 1 - kt) * p.ldb * 2 + (nl - n0 + 8) * 2);
+    bsh[i] = (int)min<int64_t>(n - nl, 8);
+  }
+  const bool edge_n = n0 + T > p.N;
+  const char* const Am = reinterpret_cast<const char*>(A + m0 * p.lda);
+  // B's base column is n0 - 8 (see boff): for n0 = 0 that is before the row,
+  // but boff is then at least 16 bytes, so no access is
+  const char* const Bn = reinterpret_cast<const char*>(B) + (n0 - 8) * 2;
+
+  u32x4_t ra[R][AP], rb[R][BP];
+  auto load = [&](int slot, int it) {
+    const int s = min(it, ns - 1);                       // past the end: the last stage again
+    const bool part = s >= nfull;
+    const char* ab = Am + (part ? at0 : kb + (int64_t)s * BK) * 2;
+    const char* bb = Bn + (kb + (int64_t)s * BK) * p.ldb * 2;
+#pragma unroll
+    for (int i = 0; i < AP; ++i)
+      ra[slot][i] = *reinterpret_cast<const u32x4_any_t*>(ab + (part ? atoff[i] : aoff[i]));
+#pragma unroll
+    for (int i = 0; i < BP; ++i)
+      rb[slot][i] = *reinterpret_cast<const u32x4_any_t*>(bb + (part ? btoff[i] : boff[i]));
+  };
+  auto put = [&](int slot, int buf, int it) {
+    if (it >= nfull) {                  // the partial stage; past it, zeros
+      const int left = it < ns ? rem : 0;
+#pragma unroll
+      for (int i = 0; i < AP; ++i) ra[slot][i] = shift_down(ra[slot][i], left ? ash[i] : 8);
+#pragma unroll
+      for (int i = 0; i < BP; ++i)
+        if (brow[i] >= left) rb[slot][i] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    if (edge_n) {
+#pragma unroll
+      for (int i = 0; i < BP; ++i) rb[slot][i] = shift_down(rb[slot][i], bsh[i]);
+    }
+    lds_char_t* const s = lds + buf * STAGE + lane * 16;
+#pragma unroll
+    for (int i = 0; i < AP; ++i)
+      *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(s + (wave * AP + i) * 1024) =
+          ra[slot][i];
+#pragma unroll
+    for (int i = 0; i < BP; ++i)
+      *reinterpret_cast<__attribute__((address_space(3))) u32x4_t*>(s + A_BYTES +
+                                                                    (wave * BP + i) * 1024) =
+          rb[slot][i];
+  };
+
+  const int wm = wave & 1, wn = wave >> 1;
+  const int lr = lane & 15, lg = lane >> 4;
+  f32x4_t acc[TT][TT];  // [n tile][m tile]: C^T tiles
+#pragma unroll
+  for (int i = 0; i < TT; ++i)
+#pragma unroll
+    for (int j = 0; j < TT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // fragments of a stage, two sets: one being multiplied, one being read
+  constexpr int KS = BK / 32;
+  u32x4_t af[2][KS][TT], bfr[2][KS][TT];
+  auto fetch = [&](int set, int buf, int ks, int q) {
+    const lds_char_t* la = lds + buf * STAGE;
+    const lds_char_t* lb = la + A_BYTES;
+    const int m = wm * (T / 2) + q * 16 + lr;
+    const int ca = (ks * 4 + lg) ^ a_swz<BK>(m);
+    af[set][ks][q] = *(const __attribute__((address_space(3))) u32x4_t*)(la + m * A_ROW + ca * 16);
+    const int k0r = ks * 32 + lg * 8 + (lr >> 2), c4 = lr & 3;
+    const int cb = (((wn * (T / 2) + q * 16) >> 3) + (c4 >> 1)) ^ b_swz_t<T>(k0r);
+    const lds_char_t* pb = lb + k0r * B_ROW + cb * 16 + (c4 & 1) * 8;
+    const u32x2_t lo = lds_read_tr16(pb), hi = lds_read_tr16(pb + 4 * B_ROW);
+    bfr[set][ks][q] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+  };
+
+  // ---- pipeline: step `it` multiplies the fragments of stage it while it
+  // reads those of stage it+1, stores stage it+2 (into the LDS stage that held
+  // stage it) and loads stage it+2+R into the registers that frees.  One
+  // barrier a step: it publishes the store and frees the LDS stage just read.
+  // Past the last stage the loads repeat it and the stores are zeros.
+  auto step = [&](int u, int it) {
+    // (fenced: the compiler would sink the fragment reads behind the MFMAs)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int tn = 0; tn < TT; ++tn) {
+        fetch((u + 1) & 1, (u + 1) & 1, ks, tn);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tm = 0; tm < TT; ++tm)
+          acc[tn][tm] = mfma16t<H>(bfr[u & 1][ks][tn], af[u & 1][ks][tm], acc[tn][tm]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ks * TT + tn == KS * TT / 2 - 1) {
+          put((u + 2) % R, u & 1, it + 2);
+          load((u + 2) % R, it + 2 + R);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    LOOM_WAIT_LGKM0();
+    barrier_nofence();
+  };
+#pragma unroll
+  for (int s = 0; s < R; ++s) load(s, s);
+  put(0, 0, 0);
+  load(0, R);
+  put(1, 1, 1);
+  load(1, R + 1);
+  LOOM_WAIT_LGKM0();
+  barrier_nofence();
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int q = 0; q < TT; ++q) fetch(0, 0, ks, q);
+  LOOM_WAIT_LGKM0();
+  barrier_nofence();
+  // (whole rounds of R: an exit in between would make the compiler wait for
+  // every load at the loop's head, and a remainder's copy of the step is more
+  // code to fetch than the zero stages it saves)
+  for (int it0 = 0; it0 < ns; it0 += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) step(u, it0 + u);
+  }
+
+  // ---- epilogue: C staged row-major (16-byte chunks XOR-swizzled by row, as
+  // in gemm_pipe_kernel) and stored as whole rows, 16 bytes per lane at any
+  // element address; a chunk that passes column N goes element by element
+  constexpr int CNC = C_ROW / 16, CPC = 16 / ES;          // chunks per row, elements per chunk
+  constexpr int CRPW = C_ROW >= 256 ? 1 : 256 / C_ROW;
+  constexpr int CSWM = (CNC < 16 ? CNC : 16) - 1;
+  auto c_swz = [](int rr) { return (rr / CRPW) & CSWM; };
+#pragma unroll
+  for (int tm = 0; tm < TT; ++tm) {
+    const int rr = wm * (T / 2) + tm * 16 + lr;
+#pragma unroll
+    for (int tn = 0; tn < TT; ++tn) {
+      const int col = wn * (T / 2) + tn * 16 + lg * 4;
+      lds_char_t* const dst =
+          lds + rr * C_ROW + (((col * ES) / 16) ^ c_swz(rr)) * 16 + (col * ES) % 16;
+      if constexpr (OUT_F32)
+        *reinterpret_cast<__attribute__((address_space(3))) f32x4_t*>(dst) = acc[tn][tm];
+      else
+        *reinterpret_cast<__attribute__((address_space(3))) u32x2_t*>(dst) = u32x2_t{
+            pack2<H>(acc[tn][tm][0], acc[tn][tm][1]), pack2<H>(acc[tn][tm][2], acc[tn][tm][3])};
+    }
+  }
+  LOOM_WAIT_LGKM0();
+  barrier_nofence();
+  typedef typename std::conditional<OUT_F32, uint32_t, uint16_t>::type elem_t;
+  elem_t* const cz = static_cast<elem_t*>(p.C) + (int64_t)z * p.zc;
+#pragma unroll
+  for (int k = 0; k < T * CNC / 256; ++k) {
+    const int idx = k * 256 + tid;
+    const int rr = idx / CNC, col = ((idx % CNC) ^ c_swz(rr)) * CPC;
+    const u32x4_t v =
+        *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(lds + idx * 16);
+    if (m0 + rr >= p.M) continue;
+    elem_t* const dst = cz + (m0 + rr) * p.ldc + n0 + col;
+    const int64_t left = p.N - (n0 + col);
+    if (left >= CPC) {
+      *reinterpret_cast<u32x4_any_t*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < CPC - 1; ++e)
+        if (e < left)
+          dst[e] = OUT_F32 ? (elem_t)v[e & 3] : (elem_t)(v[(e / 2) & 3] >> (16 * (e & 1)));
+    }
+  }
+}
+
+// Launches the ragged kernel when every K range ends at column 8 or later, N
+// is at least 8 and the per-lane offsets fit 32 bits.
+template <int T, bool H>
+bool launch_ragged(GemmParams p, bool out_f32, hipStream_t st) {
+  if (std::min(p.k_total, p.k_slab) < 8 || p.N < 8 || p.lda >= (1 << 22) || p.ldb >= (1 << 22))
+    return false;
+  p.tiles_m = (int)cdiv64(p.M, T);
+  p.tiles_n = (int)cdiv64(p.N, T);
+  const int64_t nblocks = (int64_t)p.tiles_m * p.tiles_n * p.nz;
+  if (nblocks > 0x7fffffff) return false;
+  const dim3 grid((unsigned)nblocks), block(256);
+  if (out_f32)
+    hipLaunchKernelGGL((gemm_ragged_kernel<T, true, H>), grid, block, 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_ragged_kernel<T, false, H>), grid, block, 0, st, p);
+  return true;
+}
+
 // out[e] = bf16( sum_{s ascending} G[s][e] ) -- the split-0 reduction of
 // examples/split_k_mm_gather/IR/00_from_helion_frontend.mlir:34-51.
 template <bool H>
@@ -1073,20 +1376,17 @@ __global__ void __launch_bounds__(256) splitk_reduce_scalar(const float* __restr
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool H>
-hipError_t launch_tile(const GemmParams& p, bool aligned, bool out_f32, hipStream_t st) {
-  const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * p.nz)), block(64 * WM * WN);
-  if (aligned) {
-    if (out_f32)
-      hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, true, true, H>), grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, true, false, H>), grid, block, 0, st, p);
-  } else {
-    if (out_f32)
-      hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, false, true, H>), grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, false, false, H>), grid, block, 0, st, p);
-  }
+template <int BM, int BN, int WM, int WN, bool ALIGNED, bool H>
+hipError_t launch_tile(GemmParams p, bool out_f32, hipStream_t st) {
+  p.tiles_m = (int)cdiv64(p.M, BM);
+  p.tiles_n = (int)cdiv64(p.N, BN);
+  const int64_t nblocks = (int64_t)p.tiles_m * p.tiles_n * p.nz;
+  if (nblocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+  const dim3 grid((unsigned)nblocks), block(64 * WM * WN);
+  if (out_f32)
+    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, ALIGNED, true, H>), grid, block, 0, st, p);
+  else
+    hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, ALIGNED, false, H>), grid, block, 0, st, p);
   return hipGetLastError();
 }
 
@@ -1101,15 +1401,22 @@ constexpr int kDmaBK = 32, kDmaNS = 4;
 template <bool H>
 hipError_t launch_gemm(GemmParams p, int64_t tile_m, int64_t tile_n, bool aligned, bool out_f32,
                        hipStream_t st) {
+  if (!aligned) {
+    // rows off 16-byte boundaries: the ragged kernel (its 128 tile for 256
+    // too), element loads where it cannot run
+    const bool done = tile_m == 64 ? launch_ragged<64, H>(p, out_f32, st)
+                                   : launch_ragged<128, H>(p, out_f32, st);
+    return done ? hipGetLastError() : launch_tile<64, 64, 1, 2, false, H>(p, out_f32, st);
+  }
   p.tiles_m = (int)cdiv64(p.M, tile_m);
   p.tiles_n = (int)cdiv64(p.N, tile_n);
   if (tile_m == 64) {
     if (launch_pipe<64, H>(p, aligned, out_f32, st)) return hipGetLastError();
-    return launch_tile<64, 64, 1, 2, H>(p, aligned, out_f32, st);
+    return launch_tile<64, 64, 1, 2, true, H>(p, out_f32, st);
   }
   if (tile_m == 128) {
     if (launch_pipe<128, H>(p, aligned, out_f32, st)) return hipGetLastError();
-    return launch_tile<128, 128, 2, 2, H>(p, aligned, out_f32, st);
+    return launch_tile<128, 128, 2, 2, true, H>(p, out_f32, st);
   }
   if (launch_persist<H>(p, aligned, out_f32, st)) return hipGetLastError();
   if (launch_pipe<256, H>(p, aligned, out_f32, st)) return hipGetLastError();
@@ -1124,7 +1431,7 @@ hipError_t launch_gemm(GemmParams p, int64_t tile_m, int64_t tile_n, bool aligne
       hipLaunchKernelGGL((gemm_dma_kernel<BK, NS, false, H>), grid, block, 0, st, p);
     return hipGetLastError();
   }
-  return launch_tile<256, 256, 2, 4, H>(p, aligned, out_f32, st);
+  return launch_tile<256, 256, 2, 4, true, H>(p, out_f32, st);
 }
 
 // Checks what every GEMM entry point shares.  On success *wg is the square
@@ -1185,8 +1492,8 @@ int matmul_impl(const void* x, const void* y, void* out, int64_t M, int64_t N, i
   // register-staged kernel (element stores)
   const bool al = K % 8 == 0 && N % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(out);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  (void)launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream));
-  return loom_check_launch(err, errlen, "matmul");
+  return loom_launched(launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream)), err,
+                       errlen, "matmul");
 }
 
 template <bool H>
@@ -1226,8 +1533,8 @@ int batch_matmul_impl(const void* arg0, const void* arg1, void* arg2, int64_t Bt
   const bool al =
       K % 8 == 0 && N % 8 == 0 && aligned16(arg0) && aligned16(arg1) && aligned16(arg2);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  (void)launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream));
-  return loom_check_launch(err, errlen, "batch_matmul");
+  return loom_launched(launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream)), err,
+                       errlen, "batch_matmul");
 }
 
 
@@ -1268,8 +1575,8 @@ int split_k_matmul_gather_impl(const void* a, const void* b, void* out, void* pa
   const bool al = K % 8 == 0 && N % 8 == 0 && tile_k % 8 == 0 && aligned16(a) && aligned16(b) &&
                   aligned16(partials);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  (void)launch_gemm<H>(p, wg, wg, al, true, st);
-  rc = loom_check_launch(err, errlen, "split_k_matmul_gather (slab GEMM)");
+  rc = loom_launched(launch_gemm<H>(p, wg, wg, al, true, st), err, errlen,
+                     "split_k_matmul_gather (slab GEMM)");
   if (rc) return rc;
   const int64_t MN = M * N;
   if (MN % 4 == 0 && aligned16(partials) && (reinterpret_cast<uintptr_t>(out) & 7u) == 0) {
