@@ -15,7 +15,6 @@
 //   gemm_pipe_kernel<T>  T x T tiles (256, 128, 64), one per workgroup,
 //                        software-pipelined LDS-DMA stages with the MFMA
 //                        fragments of the next stage read during this one.
-//   gemm_dma_kernel      256x256 tiles, LDS-DMA stages, K a multiple of 32.
 //   gemm_ragged_kernel<T> rows off 16-byte boundaries (K or N not a multiple of
 //                        8): 16-byte register loads at any element, the
 //                        pipelined kernels' LDS layouts.
@@ -233,22 +232,12 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// 256x256 tile, LDS-DMA pipeline.  Four waves, each owning a 128x128 block of
-// C.  Per stage, A [256][BK] and B [BK][256] are copied global -> LDS by
-// global_load_lds_dwordx4 (no staging registers; addresses clamped inside
-// each operand, the rows and columns past its extent are never stored),
-// NS stages deep.  B stays in its [k][n] layout: the MFMA
-// operand with eight consecutive k per lane comes from two ds_read_b64_tr_b16.
-// The MFMA computes C^T tiles (B^T as the row operand, A^T as the column
-// operand), so each lane ends with four consecutive columns of one row of C:
-// 8-byte (bf16) or 16-byte (fp32) stores straight from registers.
-// Swizzles (16-byte chunk index XOR a function of the row, a_swz / b_swz)
-// keep the operand reads free of bank conflicts; the DMA writes are linear
-// 1 KB blocks per instruction.
-// Each stage buffer is its own __shared__ array and the main loop is unrolled
-// by NS, so every LDS address is a constant offset; the DMAs are issued from
-// inline assembly and waited for by hand (s_waitcnt vmcnt(n) for the stage
-// needed next), with barriers that do not drain the DMAs still in flight.
+// LDS layouts of the pipelined kernels.  A stages are [T][BK], B stages
+// [BK][T], as the operands lie in memory: the MFMA operand of B with eight
+// consecutive k per lane comes from two ds_read_b64_tr_b16.  Swizzles (16-byte
+// chunk index XOR a function of the row, a_swz / b_swz) keep the operand reads
+// free of bank conflicts; the DMA writes are linear 1 KB blocks per
+// instruction.
 // ---------------------------------------------------------------------------
 // gfx950's LDS has 128 four-byte banks (512 bytes) and serves a wave's
 // ds_read_b128 / ds_read_b64_tr_b16 in two passes of 32 lanes, so the 32
@@ -273,191 +262,36 @@ LOOM_DEV int a_swz(int row) {
 // 8 ((k >> 3) & 1) put the eight pieces in distinct 32-byte slots.
 LOOM_DEV int b_swz(int k) { return (2 * (k & 3)) ^ (8 * ((k >> 3) & 1)); }
 
-template <int BK, int NS, bool OUT_F32, bool H>
-__global__ void __launch_bounds__(256) gemm_dma_kernel(GemmParams p) {
-  constexpr int BM = 256, BN = 256;
-  constexpr int A_BYTES = BM * BK * 2, B_BYTES = BK * BN * 2;
-  constexpr int A_ROWS_PER_I = 1024 / (BK * 2);   // A rows per DMA instruction
-  constexpr int A_CPR = BK / 8;                   // 16-byte chunks per A row
-  constexpr int A_INSTR = A_BYTES / 1024 / 4;     // per wave per stage
-  constexpr int B_INSTR = B_BYTES / 1024 / 4;
-  constexpr int LPW = A_INSTR + B_INSTR;          // DMA instructions per wave per stage
-  static_assert(NS >= 2 && NS <= 4, "2..4 stages");
-  static_assert(LPW * (NS - 2) <= 63, "vmcnt range");
-  __shared__ __attribute__((aligned(1024))) char sA0[A_BYTES], sB0[B_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sA1[A_BYTES], sB1[B_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sA2[NS > 2 ? A_BYTES : 16], sB2[NS > 2 ? B_BYTES : 16];
-  __shared__ __attribute__((aligned(1024))) char sA3[NS > 3 ? A_BYTES : 16], sB3[NS > 3 ? B_BYTES : 16];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  // wave-uniform by construction; readfirstlane lets the compiler know (the
-  // LDS destination of a DMA load lives in M0)
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-  // ---- which tile, which z (XCD-contiguous, grouped by 8 tile rows)
-  const int nblocks = p.tiles_m * p.tiles_n * p.nz;
-  const int bid = xcd_remap(blockIdx.x, nblocks);
-  const int per_z = p.tiles_m * p.tiles_n;
-  const int z = bid / per_z;
-  const int t = bid - z * per_z;
-  constexpr int GM = 8;
-  const int group = t / (GM * p.tiles_n);
-  const int first_m = group * GM;
-  const int gsz = min(p.tiles_m - first_m, GM);
-  const int tin = t - group * GM * p.tiles_n;
-  const int64_t m0 = (int64_t)(first_m + tin % gsz) * BM;
-  const int64_t n0 = (int64_t)(tin / gsz) * BN;
-
-  const uint16_t* A = p.A;
-  const uint16_t* B = p.B;
-  int64_t kb = 0, ke = p.k_total;
-  if (p.split) {
-    kb = (int64_t)z * p.k_slab;
-    ke = min(p.k_total, kb + p.k_slab);
-  } else {
-    A += (int64_t)z * p.za;
-    B += (int64_t)z * p.zb;
-  }
-
-  auto stageA = [&](int s) -> lds_char_t* {
-    if (s == 0) return (lds_char_t*)sA0;
-    if (s == 1) return (lds_char_t*)sA1;
-    if (s == 2) return (lds_char_t*)sA2;
-    return (lds_char_t*)sA3;
-  };
-  auto stageB = [&](int s) -> lds_char_t* {
-    if (s == 0) return (lds_char_t*)sB0;
-    if (s == 1) return (lds_char_t*)sB1;
-    if (s == 2) return (lds_char_t*)sB2;
-    return (lds_char_t*)sB3;
-  };
-
-  // ---- DMA one stage: this wave's A_INSTR + B_INSTR 1 KB blocks
-  auto issue = [&](int s, int64_t k0) {
-    const uint32_t la = lds_addr(stageA(s));
-    const uint32_t lb = lds_addr(stageB(s));
-#pragma unroll
-    for (int i = 0; i < A_INSTR; ++i) {
-      const int j = wave * A_INSTR + i;
-      const int row = j * A_ROWS_PER_I + lane / A_CPR;
-      const int c = (lane % A_CPR) ^ a_swz<BK>(row);
-      const int64_t gm = min<int64_t>(m0 + row, p.M - 1);
-      dma_load16(A + gm * p.lda + k0 + c * 8, la + j * 1024);
-    }
-#pragma unroll
-    for (int i = 0; i < B_INSTR; ++i) {
-      const int j = wave * B_INSTR + i;
-      const int row = j * 2 + lane / 32;
-      const int c = (lane % 32) ^ b_swz(row);
-      const int64_t gn = min<int64_t>(n0 + c * 8, p.N - 8);
-      dma_load16(B + (k0 + row) * p.ldb + gn, lb + j * 1024);
-    }
-  };
-
-  const int wm = wave & 1, wn = wave >> 1;
-  const int lr = lane & 15, lg = lane >> 4;
-  f32x4_t acc[8][8];  // [n tile][m tile]
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  auto compute = [&](int s) {
-    const lds_char_t* la = stageA(s);
-    const lds_char_t* lb = stageB(s);
-#pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {
-      u32x4_t af[8];
-#pragma unroll
-      for (int tm = 0; tm < 8; ++tm) {
-        // column operand A^T: lane holds A[m][32 ks + 8 lg .. +7], m = tile row lr
-        const int m = wm * 128 + tm * 16 + lr;
-        const int ch = (ks * 4 + lg) ^ a_swz<BK>(m);
-        af[tm] = *(const __attribute__((address_space(3))) u32x4_t*)(la + m * (BK * 2) + ch * 16);
-      }
-#pragma unroll
-      for (int tn = 0; tn < 8; ++tn) {
-        // row operand B^T: lane holds B[32 ks + 8 lg .. +7][n], n = tile col lr
-        const int nb = wn * 128 + tn * 16;
-        const int a = lr >> 2, c4 = lr & 3;
-        const int k0r = ks * 32 + lg * 8 + a;          // & 3 == a
-        const int ch = ((nb >> 3) + (c4 >> 1)) ^ b_swz(k0r);
-        const lds_char_t* q = lb + k0r * 512 + ch * 16 + (c4 & 1) * 8;
-        const u32x2_t lo = lds_read_tr16(q);
-        const u32x2_t hi = lds_read_tr16(q + 4 * 512);
-        const u32x4_t bf = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
-#pragma unroll
-        for (int tm = 0; tm < 8; ++tm) acc[tn][tm] = mfma16t<H>(bf, af[tm], acc[tn][tm]);
-      }
-    }
-  };
-
-  const int nk = ke > kb ? (int)((ke - kb) / BK) : 0;  // K range is a multiple of BK
-#pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < nk) issue(s, kb + (int64_t)s * BK);
-
-  for (int it0 = 0; it0 < nk; it0 += NS) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int it = it0 + s;
-      if (it < nk) {
-        // my DMA for stage `it` is done once at most the younger stages'
-        // loads are outstanding; the barrier makes everyone's visible and
-        // frees the buffer read in the previous iteration
-        const int younger = min(NS - 2, nk - 1 - it);
-        if (younger >= 2) LOOM_WAIT_VMCNT(2 * LPW);
-        else if (younger == 1) LOOM_WAIT_VMCNT(LPW);
-        else LOOM_WAIT_VMCNT(0);
-        barrier_nofence();
-        if (it + NS - 1 < nk) issue((s + NS - 1) % NS, kb + (int64_t)(it + NS - 1) * BK);
-        compute(s);
-      }
-    }
-  }
-
-  // ---- epilogue: acc[tn][tm][i] = C[m][n + i], m = tile row, n = 4 lg.
-  // The scheduling fences keep the compiler from pulling all 256 accumulators
-  // into VGPRs at once (which would set the kernel's VGPR budget).
-#pragma unroll
-  for (int tm = 0; tm < 8; ++tm) {
-    __builtin_amdgcn_sched_barrier(0);
-    const int64_t row = m0 + wm * 128 + tm * 16 + lr;
-    if (row >= p.M) continue;
-#pragma unroll
-    for (int tn = 0; tn < 8; ++tn) {
-      const int64_t col = n0 + wn * 128 + tn * 16 + lg * 4;
-      if (col >= p.N) continue;
-      const f32x4_t v = acc[tn][tm];
-      if constexpr (OUT_F32)
-        *reinterpret_cast<f32x4_t*>(static_cast<float*>(p.C) + (int64_t)z * p.zc + row * p.ldc + col) = v;
-      else
-        *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(p.C) + (int64_t)z * p.zc + row * p.ldc + col) =
-            u32x2_t{pack2<H>(v[0], v[1]), pack2<H>(v[2], v[3])};
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// Square T x T tile (T = 256, 128 or 64), software-pipelined: the production path
-// for K ranges that are whole multiples of NS*BK.  Four waves, each owning a
-// (T/2) x (T/2) block of C^T tiles; A [T][32] and B [32][T] stages arrive by
-// LDS DMA, NS deep (T 256: 4 stages of 32 KB; 128: 4 of 16 KB; 64: 8 of
-// 8 KB).  Deeper rings of the smaller tiles (8 and 16 stages, 128 KB) were
-// slower: split-K 512x512x16384 23.9 against 23.0 us, mm 1024^3 from HBM 8.0
-// against 7.6 us (4 and 2 stages: 31.9 us and 8.1 us).
-// The LDS layouts, swizzles and operand roles are those of gemm_dma_kernel
-// (and the accumulation order too: results are bitwise identical); what
-// differs is the schedule:
+// Square T x T tile (T = 256, 128 or 64), software-pipelined: the production path.
+// Four waves, each owning a (T/2) x (T/2) block of C^T tiles; A [T][32] and
+// B [32][T] stages arrive by LDS DMA (global_load_lds_dwordx4, no staging
+// registers; addresses clamped inside each operand, the rows and columns past
+// its extent are never stored), NS deep (T 256: 4 stages of 32 KB; 128: 4 of
+// 16 KB; 64: 8 of 8 KB).  Deeper rings of the smaller tiles (8 and 16 stages,
+// 128 KB) were slower: split-K 512x512x16384 23.9 against 23.0 us, mm 1024^3
+// from HBM 8.0 against 7.6 us (4 and 2 stages: 31.9 us and 8.1 us).
+// The MFMA computes C^T tiles (B^T as the row operand, A^T as the column
+// operand), so each lane ends with four consecutive columns of one row of C.
+// The DMAs are issued from inline assembly and waited for by hand (s_waitcnt
+// vmcnt(n) for the stage needed next), with barriers that do not drain the
+// DMAs still in flight.  The schedule:
 //   - the MFMA fragments of stage it+1 are read from LDS into a second
 //     register set while the MFMAs of stage it run, spread between them;
 //   - this wave's DMA for stage it+NS is folded between the MFMAs too (one
 //     per group of T/32 MFMAs), with a scalar base per stage and per-lane
 //     32-bit offsets that stay the same for every stage;
 //   - the accumulators live in AGPRs (inline-asm MFMAs, see mfma_agpr) and
-//     the loop body has no data-dependent branch: past the last stage the
-//     DMA re-reads the last stage into a buffer that is never read again;
+//     the main loop's body has no data-dependent branch: past the last stage
+//     the DMA re-reads the last stage into a buffer that is never read again;
+//   - a K range that is not a whole number of NS-stage rounds ends in a second
+//     copy of the loop that tests each step, its last stage partial (a multiple
+//     of 8 columns): the copies of what lies past the range repeat its last
+//     rows and chunks, and the fragments read from them are zeroed in both
+//     operands.  Such ranges ran on a register-staged kernel before: mm 1000^3
+//     17.7 -> 7.3 us, 512x512x800 14.6 -> 5.4, 4096x4096x4000 116 -> 104 (256
+//     tile), 16x4096x4000 54.6 -> 13.2, split-K 512x512x16000 in slabs of 1000
+//     30.0 -> 20.2;
 //   - full tiles convert every accumulator first and then store without
 //     bounds checks.
 // One barrier per stage: it publishes stage it+1 (everyone's DMA landed,
@@ -491,7 +325,7 @@ LOOM_DEV int b_swz_t(int k) {
     return b_swz(k);
 }
 
-template <int T, bool OUT_F32, bool H>
+template <int T, bool OUT_F32, bool H, bool END>
 __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
   constexpr int NS = pipe_stages<T>(), BK = 32;
   constexpr int TT = T / 32;                     // 16-wide tiles per wave dimension
@@ -536,35 +370,43 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
     A += (int64_t)z * p.za;
     B += (int64_t)z * p.zb;
   }
-  const int nk = (int)((ke - kb) / BK);   // the host guarantees nk % NS == 0, nk >= NS
+  // stages: nfull whole ones, then one of rem columns (a multiple of 8)
+  const int nfull = (int)((ke - kb) / BK), rem = END ? (int)((ke - kb) % BK) : 0;
+  const int nk = nfull + (rem != 0);
 
   // ---- per-lane DMA byte offsets (rows / columns past the operand clamped
   // inside it; what they load is never stored)
-  uint32_t aoff[A_INSTR], boff[B_INSTR];
+  // (at*, bt*: those of the partial stage, whose chunks and rows past the
+  // range repeat its last ones; the fragments read from them are zeroed)
+  uint32_t aoff[A_INSTR], boff[B_INSTR], atoff[A_INSTR], btoff[B_INSTR];
 #pragma unroll
   for (int i = 0; i < A_INSTR; ++i) {
     const int row = (wave * A_INSTR + i) * 16 + lane / 4;
     const int64_t gm = min<int64_t>(row, p.M - 1 - m0);
-    aoff[i] = (uint32_t)(gm * p.lda * 2 + ((lane % 4) ^ a_swz<BK>(row)) * 16);
+    const int c = (lane % 4) ^ a_swz<BK>(row);
+    aoff[i] = (uint32_t)(gm * p.lda * 2 + c * 16);
+    atoff[i] = (uint32_t)(gm * p.lda * 2 + min(c, rem / 8 - 1) * 16);
   }
 #pragma unroll
   for (int i = 0; i < B_INSTR; ++i) {
     const int row = (wave * B_INSTR + i) * B_RPI + lane / B_CPR;
     const int64_t gn = min<int64_t>(((lane % B_CPR) ^ b_swz_t<T>(row)) * 8, p.N - 8 - n0);
     boff[i] = (uint32_t)(row * p.ldb * 2 + gn * 2);
+    btoff[i] = (uint32_t)(min(row, rem - 1) * p.ldb * 2 + gn * 2);
   }
   const uint16_t* const Abase = A + m0 * p.lda + kb;
   const uint16_t* const Bbase = B + n0 + kb * p.ldb;
   const uint32_t la0 = lds_addr(stageA(0)), lb0 = lds_addr(stageB(0));
   auto issue = [&](int s, int stage) {
+    const bool part = END && stage >= nfull;
     const uint16_t* ab = Abase + (int64_t)stage * BK;
     const uint16_t* bb = Bbase + (int64_t)stage * BK * p.ldb;
 #pragma unroll
     for (int i = 0; i < A_INSTR; ++i)
-      dma_load16_s(aoff[i], ab, la0 + s * A_BYTES + (wave * A_INSTR + i) * 1024);
+      dma_load16_s(part ? atoff[i] : aoff[i], ab, la0 + s * A_BYTES + (wave * A_INSTR + i) * 1024);
 #pragma unroll
     for (int i = 0; i < B_INSTR; ++i)
-      dma_load16_s(boff[i], bb, lb0 + s * B_BYTES + (wave * B_INSTR + i) * 1024);
+      dma_load16_s(part ? btoff[i] : boff[i], bb, lb0 + s * B_BYTES + (wave * B_INSTR + i) * 1024);
   };
 
   // ---- fragment addresses.  A: one lane offset (tile tm moves by 1 KB; the
@@ -602,7 +444,7 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
   // ---- prologue: NS stages in flight, fragments of stage 0
   u32x4_t af[2][TT], bfr[2][TT];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) issue(s, s);
+  for (int s = 0; s < NS; ++s) issue(s, min(s, nk - 1));
   LOOM_WAIT_VMCNT((NS - 1) * LPW);
   barrier_nofence();
 #pragma unroll
@@ -611,12 +453,23 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
     const u32x2_t lo = read_b(0, q, 0), hi = read_b(0, q, 1);
     bfr[0][q] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
   }
+  // the partial stage's fragments: this lane's eight k (8 lg ..) past the
+  // range are zero in both operands
+  auto mask = [&](u32x4_t (&fa)[TT], u32x4_t (&fb)[TT]) {
+    if (8 * lg >= rem) {
+#pragma unroll
+      for (int q = 0; q < TT; ++q) fa[q] = fb[q] = u32x4_t{0u, 0u, 0u, 0u};
+    }
+  };
+  if (END && nfull == 0) mask(af[0], bfr[0]);
 
   // ---- one stage: TT*TT MFMAs on the current set; per group of TT (tile
   // tn): the next set's B fragment tn (two transposed reads) and A fragment
-  // tn, and this wave's DMA number tn for stage it+NS
-  auto step = [&](int u, int it, const u32x4_t (&fa)[TT], const u32x4_t (&fb)[TT],
+  // tn, and this wave's DMA number tn for stage it+NS.  LAST: that stage may be
+  // the partial one or past the last, and the next set may be the partial one's
+  auto step = [&](auto lastc, int u, int it, const u32x4_t (&fa)[TT], const u32x4_t (&fb)[TT],
                   u32x4_t (&na)[TT], u32x4_t (&nb)[TT]) {
+    constexpr bool LAST = decltype(lastc)::value;
     LOOM_WAIT_VMCNT((NS - 2) * LPW);
     LOOM_WAIT_LGKM0();
     barrier_nofence();
@@ -624,6 +477,7 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
     const int sd = min(it + NS, nk - 1);
     const uint16_t* ab = Abase + (int64_t)sd * BK;
     const uint16_t* bb = Bbase + (int64_t)sd * BK * p.ldb;
+    const bool part = LAST && sd >= nfull;
     u32x2_t lo[TT];
 #pragma unroll
     for (int i = 0; i < TT * TT; ++i) {
@@ -631,11 +485,12 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
       if (tm == TT / 2) {
         if (tn < A_INSTR)
           mfma_agpr_dma<H>(acc[tn][tm], fb[tn], fa[tm],
-                           la0 + (u % NS) * A_BYTES + (wave * A_INSTR + tn) * 1024, aoff[tn], ab);
+                           la0 + (u % NS) * A_BYTES + (wave * A_INSTR + tn) * 1024,
+                           part ? atoff[tn] : aoff[tn], ab);
         else
           mfma_agpr_dma<H>(acc[tn][tm], fb[tn], fa[tm],
                            lb0 + (u % NS) * B_BYTES + (wave * B_INSTR + tn - A_INSTR) * 1024,
-                           boff[tn - A_INSTR], bb);
+                           part ? btoff[tn - A_INSTR] : boff[tn - A_INSTR], bb);
       } else {
         mfma_agpr<H>(acc[tn][tm], fb[tn], fa[tm]);
       }
@@ -648,11 +503,28 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
       if (tm == 3 * TT / 4) na[tn] = read_a(sn, tn);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (LAST) {
+      if (it + 1 == nfull && rem != 0) mask(na, nb);
+    }
   };
-  for (int it0 = 0; it0 < nk; it0 += NS) {
+  // whole rounds of NS: all of them when the range is a whole number of
+  // rounds, else those whose copies are all of whole stages; then the rest
+  const int nmain = !END || rem == 0 && nk % NS == 0 ? nk : max(0, (nfull - NS) / NS * NS);
+  int it0 = 0;
+  for (; it0 < nmain; it0 += NS) {
 #pragma unroll
     for (int u = 0; u < NS; ++u)
-      step(u, it0 + u, af[u & 1], bfr[u & 1], af[(u & 1) ^ 1], bfr[(u & 1) ^ 1]);
+      step(std::false_type{}, u, it0 + u, af[u & 1], bfr[u & 1], af[(u & 1) ^ 1],
+           bfr[(u & 1) ^ 1]);
+  }
+  if constexpr (END) {
+    for (; it0 < nk; it0 += NS) {
+#pragma unroll
+      for (int u = 0; u < NS; ++u)
+        if (it0 + u < nk)
+          step(std::true_type{}, u, it0 + u, af[u & 1], bfr[u & 1], af[(u & 1) ^ 1],
+               bfr[(u & 1) ^ 1]);
+    }
   }
   LOOM_WAIT_VMCNT(0);   // the trailing re-reads land before the workgroup ends
   // every MFMA has written its accumulator before the epilogue reads them
@@ -754,19 +626,31 @@ __global__ void __launch_bounds__(256) gemm_pipe_kernel(GemmParams p) {
   }
 }
 
-// Launches the pipelined kernel when every K range is a whole number of its
-// NS*32-deep rounds (and the per-lane DMA offsets fit in 32 bits).
+// Launches the pipelined kernel on T x T tiles when the per-lane DMA offsets
+// (T rows of A, 32 rows of B) fit 32 bits.
 template <int T, bool H>
-bool launch_pipe(const GemmParams& p, bool aligned, bool out_f32, hipStream_t st) {
+bool launch_pipe(GemmParams p, bool out_f32, hipStream_t st) {
+  p.tiles_m = (int)cdiv64(p.M, T);
+  p.tiles_n = (int)cdiv64(p.N, T);
+  const int64_t nblocks = (int64_t)p.tiles_m * p.tiles_n * p.nz;
+  if (T * p.lda * 2 >= (int64_t)1 << 32 || 33 * p.ldb * 2 >= (int64_t)1 << 32 ||
+      nblocks > 0x7fffffff)
+    return false;
+  const dim3 grid((unsigned)nblocks), block(256);
+  // whole rounds on the 256 tile, which fills the register file, take the
+  // build without the second loop (2048^3: 40 us against 43 with it; the
+  // smaller tiles take the same time either way)
   constexpr int round = pipe_stages<T>() * 32;
-  const bool ok = aligned && p.k_total % round == 0 && (!p.split || p.k_slab % round == 0) &&
-                  p.lda < (1 << 22) && p.ldb < (1 << 22) && p.N >= 8;
-  if (!ok) return false;
-  const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * p.nz)), block(256);
-  if (out_f32)
-    hipLaunchKernelGGL((gemm_pipe_kernel<T, true, H>), grid, block, 0, st, p);
-  else
-    hipLaunchKernelGGL((gemm_pipe_kernel<T, false, H>), grid, block, 0, st, p);
+  auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, st, p); };
+  if constexpr (T == 256) {
+    if (p.k_total % round == 0 && p.k_slab % round == 0) {
+      if (out_f32) launch(gemm_pipe_kernel<T, true, H, false>);
+      else launch(gemm_pipe_kernel<T, false, H, false>);
+      return true;
+    }
+  }
+  if (out_f32) launch(gemm_pipe_kernel<T, true, H, true>);
+  else launch(gemm_pipe_kernel<T, false, H, true>);
   return true;
 }
 
@@ -1019,10 +903,12 @@ __global__ void __launch_bounds__(256) gemm_persist_kernel(GemmParams p, int nr)
 // evenly over one workgroup per CU (at least two each) and the pipelined
 // kernel's conditions hold; the caller falls back otherwise.
 template <bool H>
-bool launch_persist(const GemmParams& p, bool aligned, bool out_f32, hipStream_t st) {
+bool launch_persist(GemmParams p, bool out_f32, hipStream_t st) {
+  p.tiles_m = (int)cdiv64(p.M, 256);
+  p.tiles_n = (int)cdiv64(p.N, 256);
   const int cus = stream_cus(st);   // 0 when unknown: the persistent kernel is then not used
   const int64_t ntiles = (int64_t)p.tiles_m * p.tiles_n * p.nz;
-  const bool ok = aligned && !out_f32 && !p.split && cus >= 8 && cus % 8 == 0 &&
+  const bool ok = !out_f32 && !p.split && cus >= 8 && cus % 8 == 0 &&
                   p.M % 256 == 0 && p.N % 256 == 0 && p.k_total % 128 == 0 && ntiles % cus == 0 &&
                   ntiles / cus >= 2 && p.lda < (1 << 22) && p.ldb < (1 << 22) && p.ldc < (1 << 22);
   if (!ok) return false;
@@ -1394,44 +1280,21 @@ hipError_t launch_tile(GemmParams p, bool out_f32, hipStream_t st) {
 // on the smallest one covering both symbols (loom_fit_tile).
 constexpr int64_t kGemmTiles[3] = {64, 128, 256};
 
-// Depth of the DMA pipeline of the 256x256 fallback kernel: BK-deep stages,
-// NS of them (32 x 4 measured fastest of 32/64 deep, 2-4 stages).
-constexpr int kDmaBK = 32, kDmaNS = 4;
-
 template <bool H>
-hipError_t launch_gemm(GemmParams p, int64_t tile_m, int64_t tile_n, bool aligned, bool out_f32,
-                       hipStream_t st) {
+hipError_t launch_gemm(const GemmParams& p, int64_t tile, bool aligned, bool out_f32, hipStream_t st) {
   if (!aligned) {
     // rows off 16-byte boundaries: the ragged kernel (its 128 tile for 256
     // too), element loads where it cannot run
-    const bool done = tile_m == 64 ? launch_ragged<64, H>(p, out_f32, st)
-                                   : launch_ragged<128, H>(p, out_f32, st);
+    const bool done = tile == 64 ? launch_ragged<64, H>(p, out_f32, st)
+                                 : launch_ragged<128, H>(p, out_f32, st);
     return done ? hipGetLastError() : launch_tile<64, 64, 1, 2, false, H>(p, out_f32, st);
   }
-  p.tiles_m = (int)cdiv64(p.M, tile_m);
-  p.tiles_n = (int)cdiv64(p.N, tile_n);
-  if (tile_m == 64) {
-    if (launch_pipe<64, H>(p, aligned, out_f32, st)) return hipGetLastError();
-    return launch_tile<64, 64, 1, 2, true, H>(p, out_f32, st);
-  }
-  if (tile_m == 128) {
-    if (launch_pipe<128, H>(p, aligned, out_f32, st)) return hipGetLastError();
-    return launch_tile<128, 128, 2, 2, true, H>(p, out_f32, st);
-  }
-  if (launch_persist<H>(p, aligned, out_f32, st)) return hipGetLastError();
-  if (launch_pipe<256, H>(p, aligned, out_f32, st)) return hipGetLastError();
-  const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n * p.nz)), block(256);
-  // otherwise the LDS-DMA kernel needs whole BK steps in every K range
-  constexpr int BK = kDmaBK, NS = kDmaNS;
-  const bool dma = aligned && p.k_total % BK == 0 && (!p.split || p.k_slab % BK == 0);
-  if (dma) {
-    if (out_f32)
-      hipLaunchKernelGGL((gemm_dma_kernel<BK, NS, true, H>), grid, block, 0, st, p);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<BK, NS, false, H>), grid, block, 0, st, p);
+  // the binding's tile, or a smaller one where its offsets pass 32 bits
+  if (tile >= 256 && (launch_persist<H>(p, out_f32, st) || launch_pipe<256, H>(p, out_f32, st)))
     return hipGetLastError();
-  }
-  return launch_tile<256, 256, 2, 4, true, H>(p, out_f32, st);
+  if (tile >= 128 && launch_pipe<128, H>(p, out_f32, st)) return hipGetLastError();
+  if (launch_pipe<64, H>(p, out_f32, st)) return hipGetLastError();
+  return launch_tile<64, 64, 1, 2, true, H>(p, out_f32, st);
 }
 
 // Checks what every GEMM entry point shares.  On success *wg is the square
@@ -1492,7 +1355,7 @@ int matmul_impl(const void* x, const void* y, void* out, int64_t M, int64_t N, i
   // register-staged kernel (element stores)
   const bool al = K % 8 == 0 && N % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(out);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  return loom_launched(launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream)), err,
+  return loom_launched(launch_gemm<H>(p, wg, al, false, static_cast<hipStream_t>(stream)), err,
                        errlen, "matmul");
 }
 
@@ -1533,7 +1396,7 @@ int batch_matmul_impl(const void* arg0, const void* arg1, void* arg2, int64_t Bt
   const bool al =
       K % 8 == 0 && N % 8 == 0 && aligned16(arg0) && aligned16(arg1) && aligned16(arg2);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  return loom_launched(launch_gemm<H>(p, wg, wg, al, false, static_cast<hipStream_t>(stream)), err,
+  return loom_launched(launch_gemm<H>(p, wg, al, false, static_cast<hipStream_t>(stream)), err,
                        errlen, "batch_matmul");
 }
 
@@ -1575,7 +1438,7 @@ int split_k_matmul_gather_impl(const void* a, const void* b, void* out, void* pa
   const bool al = K % 8 == 0 && N % 8 == 0 && tile_k % 8 == 0 && aligned16(a) && aligned16(b) &&
                   aligned16(partials);
   if (loom_validate_only()) return loom_ok(err, errlen);
-  rc = loom_launched(launch_gemm<H>(p, wg, wg, al, true, st), err, errlen,
+  rc = loom_launched(launch_gemm<H>(p, wg, al, true, st), err, errlen,
                      "split_k_matmul_gather (slab GEMM)");
   if (rc) return rc;
   const int64_t MN = M * N;
