@@ -17,7 +17,7 @@
  * counterpart of lib/passes/lcs/src/hw_alignment.cpp:16) up to its extent, or
  * the extent itself, and runs on the smallest workgroup tile built for it
  * that covers the value (the largest built tile above them all); other values
- * are LOOM_HIP_EINVAL.  No result depends on that choice.
+ * are LOOM_HIP_EINVAL.  No result depends on that choice beyond rounding.
  *
  * Conventions shared by every entry point:
  *   - `stream` is a hipStream_t (NULL = the default stream); work is only
@@ -110,7 +110,9 @@ int loom_hip_split_k_matmul_gather(const void* a, const void* b, void* out, void
  * reference hard-codes the f16 constant 0.08837890625 at :10); `causal`
  * (not in the reference; needs Sq == Skv) hides key j from query i < j.
  * tile_m (a multiple of 16 up to Sq, or Sq) runs as the smallest workgroup
- * query tile of 64, 128, 192, 256 covering it; tile_b (<= BH) and tile_n (<= Skv, the
+ * query tile of 64, 128, 192, 256 covering it, or as 64 rows where that tile
+ * would leave CUs idle (the 64-row tile sums a row's keys in two halves, so its
+ * results differ from the others' in rounding); tile_b (<= BH) and tile_n (<= Skv, the
  * online-softmax step) are validated, the kernel streams KV in 64-key LDS
  * blocks.  D a multiple of 8 up to 256 (built for 64, 128 and 256; a
  * narrower D runs on the next one up with its padding rows zero; above 128

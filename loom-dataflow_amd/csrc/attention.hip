@@ -30,6 +30,7 @@ struct AttnParams {
   const uint16_t* q;
   uint16_t* out;
   int BH, Sq, Skv, causal, nqt;
+  int cus;     // CUs of the launch's device (0: unknown)
   int D;     // head dim: a multiple of 8, at most the kernel's D
   int koff32;  // D * Skv * 2 < 2^32: K's per-lane DMA offsets fit 32 bits
   float c2;  // scale * log2(e)
@@ -46,7 +47,11 @@ struct AttnParams {
 //   O^T[d, q]   += V^T . P^T : row operand V^T from Vs (lane r gets d = 16 dt + r,
 //                              keys 16 j0 + 4 g + 0..3 and 16 j1 + 4 g + 0..3),
 //                              exactly the keys P^T holds in lane group g.
-// Four waves of 16 QT query rows share each K/V stage.  Softmax rescaling is
+// W / KG waves of 16 QT query rows share each K/V stage.  KG 2: two waves
+// share a query tile, each taking one 32-key half of every stage, and merge at
+// the end: half the steps in a row's chain, for grids with few workgroups.
+// NSX: stages when nonzero; WPE: waves per SIMD the registers must allow.
+// Softmax rescaling is
 // lazy: a row's running max only moves (and O, l are rescaled) when a block
 // raises it by more than 8 in the log2 domain, which keeps P <= 2^8 and the
 // result exact (numerator and denominator share the stale base).
@@ -82,14 +87,15 @@ LOOM_DEV int q_swz(int lr) { return D >= 128 ? (lr & 15) : ((lr ^ (lr >> 3)) & 7
 // piece reaches past its row), issued before the block NS-1 stages ahead of
 // the one being computed and written to the same LDS position after that
 // computation; V keeps its DMA.
-template <int D, int QT, int W, bool H, bool KREG>
-__global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
+template <int D, int QT, int W, bool H, bool KREG, int KG = 1, int NSX = 0, int WPE = 1>
+__global__ void __launch_bounds__(64 * W, WPE) attention_dma_kernel(AttnParams p) {
   constexpr int KB = 64;                        // keys per stage
+  static_assert(KG == 1 || KG == 2, "a stage has two 32-key halves");
   // stages: three of 32 KB (K and V) up to D 128; two of 64 KB at D 256
   // (a fourth 32 KB stage measured 2% slower: causal B4 H32 S4096 572
   // against 561 us; two stages 554-557 us, equal within box noise)
-  constexpr int NS = D > 128 ? 2 : 3;
-  constexpr int BQ = 16 * QT * W;               // queries per workgroup
+  constexpr int NS = NSX ? NSX : (D > 128 ? 2 : 3);
+  constexpr int BQ = 16 * QT * W / KG;          // queries per workgroup
   constexpr int K_BYTES = D * KB * 2, V_BYTES = KB * D * 2;
   constexpr int K_INSTR = K_BYTES / 1024 / W;   // DMA instructions per wave per stage
   constexpr int V_INSTR = V_BYTES / 1024 / W;
@@ -114,6 +120,7 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int qw = wave / KG, kh = wave % KG;     // query rows and key half of this wave
   const int r = lane & 15, g = lane >> 4;
   const int a4 = r >> 2, c4 = r & 3;            // transposed-read lane roles
 
@@ -247,7 +254,7 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
   // ---- Q^T operands: lane holds q[q0w + 16 qt + r][32 ds + 8 g .. +7] times
   // scale * log2(e), rounded to bf16, so scores come out in the log2 domain
   // (zero past Dr)
-  const int q0w = q0 + 16 * QT * wave;
+  const int q0w = q0 + 16 * QT * qw;
   u32x4_t qf[DSTEPS][QT];
   auto q_operand = [&](int qt, int ds, u32x4_t raw) {
     if (ds * 32 + g * 8 >= Dr) raw = u32x4_t{0u, 0u, 0u, 0u};
@@ -287,13 +294,14 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
   auto compute = [&](int s, int blk) {
     const int kv0 = blk * KB;
     // a wave whose queries all precede the block sees only masked keys
-    if (p.causal && kv0 > q0w + 16 * QT - 1) return;
+    if (p.causal && kv0 + 32 * kh > q0w + 16 * QT - 1) return;
     const lds_char_t* ks = stK(s);
     const lds_char_t* vs = stV(s);
     const bool edge = kv0 + KB > Skv || (p.causal && kv0 + KB - 1 > q0w);
     // two 32-key halves, each a softmax step of its own
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int hh = 0; hh < 2 / KG; ++hh) {
+      const int h = KG == 1 ? hh : kh;
       // ---- S^T = K^T Q^T - m; st[j][qt][i] = score of key kv0 + 32 h + 16 j + 4 g + i
       f32x4_t st[2][QT];
 #pragma unroll
@@ -344,14 +352,19 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
           for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[j][qt][i]);
         lmax[qt] = mx;
         big |= mx > 8.f;
+        if constexpr (KG == 2) big |= lacc[qt][0] == 0.f;
       }
-      const bool first = blk == 0 && h == 0;
+      // (KG 2: a row's first step is the first in which its half held a key
+      // of finite score, until which l is zero, so that the base is not set by
+      // a half without one)
+      bool first = KG == 1 && blk == 0 && hh == 0;
       if (first || __builtin_amdgcn_ballot_w64(big) != 0) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
           float mx = lmax[qt];
           mx = fmaxf(mx, __shfl_xor(mx, 16));
           mx = fmaxf(mx, __shfl_xor(mx, 32));
+          if constexpr (KG == 2) first = lacc[qt][0] == 0.f;
           // the first step sets m (O and l are still zero); later ones only raise it
           const float shift = first ? (mx == -INFINITY ? 0.f : mx) : fmaxf(mx, 0.f);
           if (!first) {
@@ -413,7 +426,7 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
             // this wave's Q^T operands from the Q region (landed with stage 0)
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-              const int lr = 16 * QT * wave + 16 * qt + r;
+              const int lr = 16 * QT * qw + 16 * qt + r;
 #pragma unroll
               for (int ds = 0; ds < DSTEPS; ++ds)
                 q_operand(qt, ds, *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(
@@ -437,6 +450,40 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
     }
   }
 
+  // ---- KG 2: the pair's second wave hands its state over through the idle
+  // stages (lane by lane: both hold the same rows and columns) and is done; a
+  // half that saw no key (l = 0) takes no part
+  if constexpr (KG == 2) {
+    constexpr int SLOT = QT * (DT + 1) * 64;    // f32x4 per wave: O, then (l, m)
+    static_assert(W / 2 * SLOT * 16 <= NS * STAGE, "merge area");
+    LOOM_WAIT_VMCNT(0);
+    barrier_nofence();
+    f32x4_t* const mg = reinterpret_cast<f32x4_t*>(smem) + qw * SLOT + lane;
+    if (kh == 1) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) mg[(qt * (DT + 1) + dt) * 64] = ot[dt][qt];
+        mg[(qt * (DT + 1) + DT) * 64] = f32x4_t{lacc[qt][0], m_run[qt], 0.f, 0.f};
+      }
+    }
+    LOOM_WAIT_LGKM0();
+    barrier_nofence();
+    if (kh == 1) return;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const f32x4_t lm = mg[(qt * (DT + 1) + DT) * 64];
+      const float l0 = lacc[qt][0], l1 = lm[0], m0 = m_run[qt], m1 = lm[1];
+      const float M = l0 != 0.f ? (l1 != 0.f ? fmaxf(m0, m1) : m0) : m1;
+      const float f0 = l0 != 0.f ? fast_exp2(m0 - M) : 0.f;
+      const float f1 = l1 != 0.f ? fast_exp2(m1 - M) : 0.f;
+      lacc[qt][0] = l0 * f0 + l1 * f1;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+        ot[dt][qt] = ot[dt][qt] * f0 + mg[(qt * (DT + 1) + dt) * 64] * f1;
+    }
+  }
+
   // ---- out = acc / l; ot[dt][qt][i] is d = 16 dt + 4 g + i of query q0w + 16 qt + r.
   // With D <= 128 and rows of exactly D, each wave stages its rows in its
   // own slice of the Q region (nothing else touches it after the first
@@ -447,7 +494,7 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const float inv = 1.f / lacc[qt][0];
-        const int lr = 16 * QT * wave + 16 * qt + r;
+        const int lr = 16 * QT * qw + 16 * qt + r;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           const f32x4_t o = ot[dt][qt];
@@ -462,7 +509,7 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
 #pragma unroll
       for (int k = 0; k < 16 * QT * CPR / 64; ++k) {
         const int idx = k * 64 + lane;
-        const int lr = 16 * QT * wave + idx / CPR, cp = idx % CPR;
+        const int lr = 16 * QT * qw + idx / CPR, cp = idx % CPR;
         const u32x4_t v = *reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(
             sQ + lr * QROW + cp * 16);
         if (q0 + lr < Sq)
@@ -490,23 +537,50 @@ __global__ void __launch_bounds__(64 * W) attention_dma_kernel(AttnParams p) {
   }
 }
 
+// The workgroup query tile a binding's tile (64 .. 256) runs on: 64 rows where
+// the larger tile would leave CUs idle or uneven, else the binding's own.
+// The large tiles read each K/V stage once for up to four times the rows, but
+// a workgroup of 256 rows takes about 1.9 us per 64-key block (one fits a CU)
+// where 64 rows take 0.65, two workgroups to a CU: the line lies where their
+// rounds cost the same, at two workgroups of 64 rows per CU, and at four in a
+// causal grid, whose heaviest tile a large tile's time follows.  BH32 D128
+// S1000: causal 33 us on 256 rows, 19 on 64 (15 with BH8); not causal 33 and
+// 26; S2048: causal 61 and 49, not causal (four per CU) 67 and 86; BH128
+// S1024 causal (eight per CU) 50 and 56.  Above D 128 the large tile is 128
+// rows and the line at one workgroup per CU (BH8 S1000 causal 39 and 27).
+int64_t query_tile(int64_t tile, int64_t BH, int64_t Sq, int64_t D, bool causal, int cus) {
+  const int64_t per_cu = D > 128 ? 1 : causal ? 4 : 2;
+  return BH * cdiv64(Sq, 64) <= per_cu * cus ? 64 : tile;
+}
+
 template <bool H, bool KREG>
-void launch_attention(const AttnParams& p, int64_t D, int64_t tile_m, hipStream_t st) {
+void launch_attention(AttnParams p, int64_t D, int64_t tile_m, hipStream_t st) {
+  tile_m = query_tile(tile_m, p.BH, p.Sq, D, p.causal != 0, p.cus);
+  p.nqt = (int)cdiv64(p.Sq, tile_m);
   const dim3 grid((unsigned)(p.BH * p.nqt)), b4(256), b8(512);
+  auto launch = [&](auto kern, dim3 block) { hipLaunchKernelGGL(kern, grid, block, 0, st, p); };
   if (D == 256) {   // one 16-row query tile per wave: 64 or 128 queries
-    if (tile_m == 64) hipLaunchKernelGGL((attention_dma_kernel<256, 1, 4, H, KREG>), grid, b4, 0, st, p);
-    else hipLaunchKernelGGL((attention_dma_kernel<256, 1, 8, H, KREG>), grid, b8, 0, st, p);
+    if (tile_m == 64) launch(attention_dma_kernel<256, 1, 8, H, KREG, 2>, b8);
+    else launch(attention_dma_kernel<256, 1, 8, H, KREG>, b8);
     return;
   }
+  // 64 rows: eight waves, two to a query tile (KG 2), over two stages, so that
+  // two workgroups fit a CU (D 128, BH32 S2048 causal: 49 us, against 79 with
+  // four waves and three stages and 53 with four waves and two); at D 64
+  // and more than two workgroups per CU four waves, of which four fit (BH128
+  // S512 causal 10.9 against 13.4 us, but BH32 S333 x 1003 15.2 against 12.0)
   switch ((D == 128 ? 10 : 0) + (int)(tile_m / 64)) {
-    case 11: hipLaunchKernelGGL((attention_dma_kernel<128, 1, 4, H, KREG>), grid, b4, 0, st, p); break;
-    case 12: hipLaunchKernelGGL((attention_dma_kernel<128, 1, 8, H, KREG>), grid, b8, 0, st, p); break;
-    case 13: hipLaunchKernelGGL((attention_dma_kernel<128, 3, 4, H, KREG>), grid, b4, 0, st, p); break;
-    case 14: hipLaunchKernelGGL((attention_dma_kernel<128, 2, 8, H, KREG>), grid, b8, 0, st, p); break;
-    case 1: hipLaunchKernelGGL((attention_dma_kernel<64, 1, 4, H, KREG>), grid, b4, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((attention_dma_kernel<64, 1, 8, H, KREG>), grid, b8, 0, st, p); break;
-    case 3: hipLaunchKernelGGL((attention_dma_kernel<64, 3, 4, H, KREG>), grid, b4, 0, st, p); break;
-    default: hipLaunchKernelGGL((attention_dma_kernel<64, 2, 8, H, KREG>), grid, b8, 0, st, p); break;
+    case 11: launch(attention_dma_kernel<128, 1, 8, H, KREG, 2, 2, 2>, b8); break;
+    case 12: launch(attention_dma_kernel<128, 1, 8, H, KREG>, b8); break;
+    case 13: launch(attention_dma_kernel<128, 3, 4, H, KREG>, b4); break;
+    case 14: launch(attention_dma_kernel<128, 2, 8, H, KREG>, b8); break;
+    case 1:
+      if (grid.x <= 2u * p.cus) launch(attention_dma_kernel<64, 1, 8, H, KREG, 2, 2, 2>, b8);
+      else launch(attention_dma_kernel<64, 1, 4, H, KREG, 1, 2>, b4);
+      break;
+    case 2: launch(attention_dma_kernel<64, 1, 8, H, KREG>, b8); break;
+    case 3: launch(attention_dma_kernel<64, 3, 4, H, KREG>, b4); break;
+    default: launch(attention_dma_kernel<64, 2, 8, H, KREG>, b8); break;
   }
 }
 
@@ -528,8 +602,7 @@ int attention_impl(const void* k, const void* v, const void* q, void* out, int64
     return loom_fail(err, errlen, LOOM_EINVAL, "attention: causal needs Sq == Skv");
   // tile_m is bounded by Sq (natural_ub) and runs on the smallest built
   // query tile covering it (the largest above them: 256, or 128 for head dims
-  // above 128); a query row's result does not depend on the workgroup that
-  // holds it
+  // above 128), or on 64 rows (query_tile)
   static const int64_t kQTiles[4] = {64, 128, 192, 256};
   const int64_t wm = loom_fit_tile(tile_m, Sq, kQTiles, D > 128 ? 2 : 4);
   if (wm == 0)
@@ -568,12 +641,12 @@ int attention_impl(const void* k, const void* v, const void* q, void* out, int64
   p.Sq = (int)Sq;
   p.Skv = (int)Skv;
   p.causal = causal ? 1 : 0;
-  p.nqt = (int)cdiv64(Sq, tile_m);
   p.D = (int)D;
   p.koff32 = loom_prod_le({D, Skv, 2}, 0xffffffffll) ? 1 : 0;
   p.c2 = scale * 1.4426950408889634f;
   if (loom_validate_only()) return loom_ok(err, errlen);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  p.cus = stream_cus(st);
   // the kernel built for 64, 128 or 256 (the next one up) runs any narrower D
   const int64_t Dk = D <= 64 ? 64 : D <= 128 ? 128 : 256;
   if (kreg) launch_attention<H, true>(p, Dk, tile_m, st);

@@ -1,0 +1,91 @@
+"""The attention kernels on both sides of the rule that picks the workgroup's
+query tile: grids large enough that a binding's own tile (128, 192, 256) runs,
+and small ones, which run as 64 rows whose keys two waves share.  Sampled heads
+against the CPU oracle, at attention's bar (tests/test_gpu_parity.py).
+"""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from oracle import from_bf16, to_bf16
+from tests.conftest import assert_close
+from tests.test_gpu_parity import ATTN_TOL, dev, host, rng_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lh():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import loom_hip
+    return loom_hip
+
+
+def _check(lh, BH, Sq, Skv, D, causal, tile_m, heads):
+    rng = np.random.default_rng(BH + 7 * Sq + Skv + D)
+    k, v, q = rng_bf16(rng, (BH, D, Skv)), rng_bf16(rng, (BH, Skv, D)), rng_bf16(rng, (BH, Sq, D))
+    print(f"attention tile BH{BH} Sq{Sq} Skv{Skv} D{D} causal={causal} tile {tile_m}", flush=True)
+    got = from_bf16(host(lh.attention(dev(k), dev(v), dev(q), causal=causal, tile_m=tile_m)))
+    h = list(heads)
+    ref = from_bf16(oracle.attention(k[h], v[h], q[h], 1 / math.sqrt(D), causal, 1, 64, 64))
+    assert_close(got[h], ref, **ATTN_TOL, what=f"tile {tile_m} BH{BH} Sq{Sq} Skv{Skv} D{D} {causal}")
+
+
+# more than four workgroups of 64 rows per CU of 256
+@pytest.mark.parametrize("D,tile_m", [(64, 64), (64, 128), (64, 192), (64, 256), (72, 128),
+                                      (128, 64), (128, 128), (128, 192), (128, 256), (200, 128)])
+@pytest.mark.parametrize("Sq,Skv,causal", [(270, 270, True), (264, 264, True), (260, 100, False),
+                                           (257, 61, False)])
+def test_large_grids_run_the_bound_tile(lh, D, tile_m, Sq, Skv, causal):
+    _check(lh, 216, Sq, Skv, D, causal, tile_m, (0, 101, 215))
+
+
+# one to four workgroups of 64 rows per CU, and the rule's edges (256, 512 and
+# 1024 of them on 256 CUs)
+@pytest.mark.parametrize("BH,Sq,Skv,D,causal", [
+    (3, 300, 300, 128, True), (64, 256, 256, 128, True), (128, 256, 264, 128, False),
+    (129, 256, 264, 128, False), (256, 250, 250, 64, True), (129, 256, 40, 64, False),
+    (64, 256, 72, 256, False), (2, 130, 33, 128, False), (2, 64, 32, 128, False),
+    (2, 70, 31, 64, False), (1, 1, 1, 128, False), (2, 96, 96, 256, True)])
+def test_small_grids(lh, BH, Sq, Skv, D, causal):
+    _check(lh, BH, Sq, Skv, D, causal, min(256, Sq), range(0, BH, max(1, BH // 3)))
+
+
+@pytest.mark.parametrize("hidden", [(32, 64), (0, 32), (0, 64), (64, 128)])
+def test_halves_of_infinite_scores(lh, hidden):
+    """Keys of -inf score (an infinite k against a positive q) over one half
+    of a stage or all of it, and finite scores far below zero elsewhere: the
+    half's base is set by its first finite score."""
+    D, S = 64, 160
+    rng = np.random.default_rng(9)
+    q = np.zeros((1, 70, D), np.float32)
+    q[:, :, 0] = 8.0
+    q[:, :, 1:] = rng.standard_normal((1, 70, D - 1))
+    k = rng.standard_normal((1, D, S)).astype(np.float32)
+    k[:, 0, :] = -600.0
+    k[:, 0, hidden[0]:hidden[1]] = -np.inf
+    v = rng.standard_normal((1, S, D)).astype(np.float32)
+    k, v, q = to_bf16(k), to_bf16(v), to_bf16(q)
+    got = from_bf16(host(lh.attention(dev(k), dev(v), dev(q))))
+    s = (from_bf16(q)[0].astype(np.float64) @ from_bf16(k)[0].astype(np.float64)) / math.sqrt(D)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = (p / p.sum(-1, keepdims=True)) @ from_bf16(v)[0].astype(np.float64)
+    # every score shares the offset -600 * 8 / 8 = -600 log-units; q is scaled
+    # and rounded to bf16 once, which moves a score by up to 2^-9 of its terms'
+    # sum (about 600 * 2^-9 = 1.2 common to all keys, and 2^-9 * sum |q k| / 8
+    # between them): the common part cancels
+    assert_close(got[0], ref, atol=3e-2, rtol=2e-2, what=f"hidden {hidden}")
+
+
+def test_nan_reaches_the_row(lh):
+    """A NaN in either half of the keys makes every row NaN."""
+    rng = np.random.default_rng(10)
+    for key in (5, 40, 100):
+        k, v, q = rng_bf16(rng, (1, 64, 128)), rng_bf16(rng, (1, 128, 64)), rng_bf16(rng, (1, 64, 64))
+        kt = dev(k)
+        kt[0, 3, key] = float("nan")
+        assert torch.isnan(lh.attention(kt, dev(v), dev(q))).all(), key
