@@ -15,17 +15,19 @@
 // O^T += V^T . P^T run on MFMA and the kernel stays bound by the stream.
 // One workgroup (4 waves) per (batch, split, group of 32 query heads):
 //   - decode_dma_kernel (S a multiple of 8, or any S above D 128 or 32
-//     heads with K staged through registers; 4 waves for up to 32 heads, 8
+//     heads or in splits up to 512 keys, with K staged through registers; 4 waves for up to 32 heads, 8
 //     for 64): K and V stream through a ring of LDS-DMA stages (four, two at
 //     D 256) and reach the MFMAs by transposed LDS reads (described at the
 //     kernel);
-//   - decode_split_kernel (other S, up to 32 heads and D 128): raw buffer loads straight into
+//   - decode_split_kernel (other S, up to 32 heads and D 128, splits above 512
+//     keys): raw buffer loads straight into
 //     registers, MFMA operands built by register transposes (v_perm_b32),
 //     keys permuted inside a block and the permutation undone only where
 //     results are addressed (softmax and P.V do not depend on key order).
 // Softmax runs in the log2 domain in fp32.  The waves' partial states merge
 // through LDS into (lse_s, o_s), exactly the reference's gathered tensors;
-// decode_combine_kernel performs the split-0 combine.
+// decode_combine_kernel or, for many splits,
+// decode_combine_row_kernel performs the split-0 combine.
 // Any head dim that is a multiple of 8 up to 128 runs on the kernels built
 // for 64 or 128, and up to 256 on the LDS-DMA kernel built for 256: K rows
 // and q elements past it are zeros (copied from zeros, or read past the
@@ -55,10 +57,9 @@ struct DecodeParams {
 
 // Split-0 combine of the reference (:147-199): M = max_s lse_s,
 // w_s = exp(lse_s - M) / sum_s exp(lse_s - M), out = sum_s w_s o_s (ascending
-// s).  One thread per two consecutive d of one (b, head): every split's lse
-// and o loads are independent and issued together (in chunks of CH splits:
-// 8 when there are at most 8, else 16), so the combine costs about one
-// memory round trip.
+// s).  Up to CH splits (8 or 16): one thread per two consecutive d of one
+// (b, head), every split's lse and o loads independent and issued together,
+// so the combine costs about one memory round trip.
 template <bool F16, int CH>
 __global__ void __launch_bounds__(256) decode_combine_kernel(DecodeParams p) {
   const int D = p.D;
@@ -69,37 +70,95 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(DecodeParams p) {
   if (bh >= BH) return;
   const int d = (int)(t % TPR) * 2;
   const int ns = p.ns;
-  // every load of a chunk of CH splits is issued before any is used; across
-  // chunks the running max moves and the sums rescale (one chunk at BASELINE
-  // shapes, so one memory round trip)
-  float M = -INFINITY, den = 0.f, a0 = 0.f, a1 = 0.f;
-  for (int c0 = 0; c0 < ns; c0 += CH) {
-    float l[CH];
-    f32x2_t o[CH];
+  float l[CH];
+  f32x2_t o[CH];
 #pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const int64_t s = min(c0 + u, ns - 1);   // clamped: weight 0 past the end
-      l[u] = p.lse[s * BH + bh];
-      o[u] = *reinterpret_cast<const f32x2_t*>(p.o + (s * BH + bh) * D + d);
-    }
-    float mc = M;
+  for (int u = 0; u < CH; ++u) {
+    const int64_t s = min(u, ns - 1);   // clamped: weight 0 past the end
+    l[u] = p.lse[s * BH + bh];
+    o[u] = *reinterpret_cast<const f32x2_t*>(p.o + (s * BH + bh) * D + d);
+  }
+  float M = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < CH; ++u) mc = fmaxf(mc, l[u]);
-    const float r = expf(M - mc);   // 0 on the first chunk (M = -inf)
-    den *= r;
-    a0 *= r;
-    a1 *= r;
-    M = mc;
+  for (int u = 0; u < CH; ++u) M = fmaxf(M, l[u]);
+  float den = 0.f, a0 = 0.f, a1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < CH; ++u) {
-      const float w = c0 + u < ns ? expf(l[u] - M) : 0.f;
-      den += w;
-      a0 += w * o[u][0];
-      a1 += w * o[u][1];
-    }
+  for (int u = 0; u < CH; ++u) {
+    const float w = u < ns ? expf(l[u] - M) : 0.f;
+    den += w;
+    a0 += w * o[u][0];
+    a1 += w * o[u][1];
   }
   const float inv = 1.f / den;
   *reinterpret_cast<uint32_t*>(p.out + bh * D + d) = pack2<F16>(a0 * inv, a1 * inv);
+}
+
+// The combine of many splits: one workgroup per (b, head) row, its threads in
+// groups of D / 4 (four d each), group y taking splits y, y + NG, ...  A thread
+// issues the loads of CH of its splits at a time, so up to CH NG splits (64 at
+// D 128, 128 at D 64) cost one memory round trip, where a thread that walks
+// them 16 at a time takes one for every 16 and leaves most CUs idle when there
+// are few rows.  The groups' (max, sum, partial row) meet in LDS.  Whole call,
+// H32 D128 in 64-key splits: B1 S4096 13.2 -> 8.2 us, S16384 35 -> 13.3, B4
+// S4096 15.5 -> 10.7.
+template <bool F16>
+__global__ void __launch_bounds__(256) decode_combine_row_kernel(DecodeParams p) {
+  constexpr int CH = 8, NGMAX = 64;
+  __shared__ f32x4_t s_acc[256];
+  __shared__ float s_m[NGMAX], s_den[NGMAX];
+  const int D = p.D, ns = p.ns;
+  const int TPR = D / 4, NG = min(256 / TPR, NGMAX);
+  const int64_t BH = (int64_t)p.B * p.H, bh = blockIdx.x;
+  const int grp = (int)threadIdx.x / TPR, d = ((int)threadIdx.x % TPR) * 4;
+  float M = -INFINITY, den = 0.f;
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (grp < NG) {
+    for (int s0 = grp; s0 < ns; s0 += CH * NG) {
+      float l[CH];
+      f32x4_t o[CH];
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const int64_t s = min(s0 + u * NG, ns - 1);   // clamped: weight 0 past the end
+        l[u] = p.lse[s * BH + bh];
+        o[u] = *reinterpret_cast<const f32x4_t*>(p.o + (s * BH + bh) * D + d);
+      }
+      float mc = M;
+#pragma unroll
+      for (int u = 0; u < CH; ++u)
+        if (s0 + u * NG < ns) mc = fmaxf(mc, l[u]);
+      const float r = expf(M - mc);   // 0 on the first chunk (M = -inf)
+      den *= r;
+      acc *= r;
+      M = mc;
+#pragma unroll
+      for (int u = 0; u < CH; ++u) {
+        const float w = s0 + u * NG < ns ? expf(l[u] - M) : 0.f;
+        den += w;
+        acc += o[u] * w;
+      }
+    }
+    s_acc[threadIdx.x] = acc;
+    if (d == 0) {
+      s_m[grp] = M;
+      s_den[grp] = den;
+    }
+  }
+  __syncthreads();
+  if (grp != 0) return;
+  // groups past the splits (ns < NG) hold den = 0 and take no part
+  const int ng = min(NG, ns);
+  float Mt = -INFINITY;
+  for (int y = 0; y < ng; ++y) Mt = fmaxf(Mt, s_m[y]);
+  float dt = 0.f;
+  f32x4_t at = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int y = 0; y < ng; ++y) {
+    const float w = expf(s_m[y] - Mt);
+    dt += s_den[y] * w;
+    at += s_acc[y * TPR + (int)threadIdx.x] * w;
+  }
+  const float inv = 1.f / dt;
+  *reinterpret_cast<u32x2_t*>(p.out + bh * D + d) =
+      u32x2_t{pack2<F16>(at[0] * inv, at[1] * inv), pack2<F16>(at[2] * inv, at[3] * inv)};
 }
 
 // ---------------------------------------------------------------------------
@@ -786,15 +845,18 @@ int flash_decode_impl(const void* k, const void* v, const void* q, void* out,
   const bool d128 = D > 64;
   // More than 32 query heads: 8-wave workgroups of 64 heads, so K and V are
   // streamed once per 64 heads, not per 32 (B32 H48 D128 S8192: 33.2 us
-  // against 52.2).  S not a multiple of 8: the register kernel up to 32
-  // heads and D 128 (B32 H32 D128 S8190: 35 us against 47 with K staged
-  // through registers into the LDS-DMA kernel); that KREG form for more
-  // heads (H48 S8191: 38.9 us against the register kernel's 60.1, which
-  // takes 32 heads per pass) and above D 128, where the register kernel is
-  // not built
+  // against 52.2).  S not a multiple of 8: long splits up to 32 heads and
+  // D 128 take the register kernel (tile_s 1024, B32 H32 D128 S8191: 36.0 us
+  // against 38.7 with K staged through registers into the LDS-DMA kernel, H16
+  // 32 against 38); its four waves take a 64-key block each, so up to 512
+  // keys a split that KREG form is faster (tile_s 512, the same shape: 46.7 ->
+  // 35.6; B1 S4097 in 64-key splits 14.2 -> 9.4).  More heads take KREG too
+  // (H48 S8191: 38.9 us against the register kernel's 60.1, which takes 32
+  // heads per pass), and so does D above 128, where the register kernel is not
+  // built
   const bool kreg = S % 8 != 0;
   const bool wide = H > 32;
-  if (!kreg || D > 128 || wide) {
+  if (!kreg || D > 128 || wide || tile_s <= 512) {
     if (D > 128) launch_dma<256, F16>(p, kreg, wide, st);
     else if (d128) launch_dma<128, F16>(p, kreg, wide, st);
     else launch_dma<64, F16>(p, kreg, wide, st);
@@ -807,9 +869,17 @@ int flash_decode_impl(const void* k, const void* v, const void* q, void* out,
   }
   int rc = loom_check_launch(err, errlen, "flash_decode (split)");
   if (rc) return rc;
+  // Few splits, one thread per two d of a row; many, one workgroup per row.
+  // At 9 to 16 splits the former while its threads cover the CUs (B32 H32 D128
+  // S8192 in 16 splits: 32.7 against 33.5 us), the latter for fewer rows (B4
+  // H32 S1025 in 17: 10.3 -> 8.7)
   const dim3 cgrid((unsigned)cdiv64(B * H * D / 2, 256)), cblock(256);
-  if (p.ns <= 8) hipLaunchKernelGGL((decode_combine_kernel<F16, 8>), cgrid, cblock, 0, st, p);
-  else hipLaunchKernelGGL((decode_combine_kernel<F16, 16>), cgrid, cblock, 0, st, p);
+  if (p.ns <= 8)
+    hipLaunchKernelGGL((decode_combine_kernel<F16, 8>), cgrid, cblock, 0, st, p);
+  else if (p.ns <= 16 && (int64_t)cgrid.x >= 256)
+    hipLaunchKernelGGL((decode_combine_kernel<F16, 16>), cgrid, cblock, 0, st, p);
+  else
+    hipLaunchKernelGGL((decode_combine_row_kernel<F16>), dim3((unsigned)(B * H)), cblock, 0, st, p);
   return loom_check_launch(err, errlen, "flash_decode (combine)");
 }
 
