@@ -1,0 +1,113 @@
+"""The short way of a well-formed call (loom_hip._plan, _prologue_plan) accepts
+exactly the signatures that the full checks accept, and gives the same
+extents, tiles and output shapes (CPU only: signatures are types and shapes)."""
+import itertools
+
+import pytest
+import torch
+
+import loom_hip as lh
+
+bf, f16, f32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _meta(dtype, shape):
+    return torch.empty(shape, dtype=dtype, device="meta")
+
+
+def _full(func, tensors, given):
+    """Extents, tiles, type and output shape by the full checks."""
+    e, _ = lh._elt(tensors[1 if func == "helion_mamba2_chunk_scan_kernel" else 0])
+    dims = lh._dims_of(func, tensors)
+    spec = lh._SPECS[func](*dims)
+    side = f32 if e == bf else f16
+    for t, (name, kind, shape) in zip(tensors, spec):
+        lh._check_form(t, name, e if kind == "e" else side, shape)
+    return tuple(dims), tuple(lh._tiles(func, dims, **given)), e, tuple(spec[-1][2])
+
+
+CALLS = {
+    "matmul": ([(64, 32), (32, 48)], ("tile_m", "tile_n", "tile_k")),
+    "batch_matmul": ([(2, 64, 32), (2, 32, 48)], ("tile_b", "tile_m", "tile_n", "tile_k")),
+    "split_k_matmul_gather": ([(64, 512), (512, 48)], ("tile_m", "tile_n", "tile_k")),
+    "attention": ([(2, 64, 100), (2, 100, 64), (2, 90, 64)], ("tile_b", "tile_m", "tile_n")),
+    "flash_decode": ([(2, 64, 100), (2, 100, 64), (2, 9, 64)], ("tile_b", "tile_s", "tile_n")),
+    "helion_mamba2_chunk_scan_kernel": (
+        [(1, 2, 1, 64, 64), (1, 4, 128, 32), (1, 4, 2, 64), (1, 4, 2, 64), (1, 1, 128, 64), (4,),
+         (1, 2, 4, 64, 32)], ("tile_b", "tile_h", "tile_c", "tile_m", "tile_n", "tile_k")),
+}
+
+
+def _variants(shapes):
+    """The signature itself, each extent of each input one off, a dimension
+    more or fewer, and every choice of one input's type."""
+    yield shapes, None
+    for i, s in enumerate(shapes):
+        for d in range(len(s)):
+            yield [t if j != i else s[:d] + (s[d] + 1,) + s[d + 1:] for j, t in enumerate(shapes)], None
+        yield [t if j != i else s[:-1] for j, t in enumerate(shapes)], None
+        yield [t if j != i else (1,) + s for j, t in enumerate(shapes)], None
+        for dt in (bf, f16, f32):
+            yield shapes, (i, dt)
+
+
+@pytest.mark.parametrize("func", CALLS)
+@pytest.mark.parametrize("base", [bf, f16, f32])
+@pytest.mark.parametrize("tile", [None, 16])
+def test_plans_match_the_full_checks(func, base, tile):
+    shapes0, symbols = CALLS[func]
+    given = {s: (1 if s in ("tile_b", "tile_h", "tile_c") else tile) if tile else None
+             for s in symbols}
+    accepted = 0
+    for shapes, change in _variants(shapes0):
+        sides = {2, 3, 5, 6} if func.startswith("helion") else set()
+        types = [f32 if i in sides and base == bf else base for i in range(len(shapes))]
+        if change:
+            types[change[0]] = change[1]
+        tensors = [_meta(t, s) for t, s in zip(types, shapes)]
+        sig = tuple(itertools.chain.from_iterable((t.dtype, t.shape) for t in tensors))
+        plan = lh._plan(func, sig, tuple(given.items()))
+        try:
+            want = _full(func, tensors, given)
+        except (ValueError, TypeError, RuntimeError):
+            want = None
+        assert (plan is None) == (want is None), (func, shapes, types)
+        if plan:
+            accepted += 1
+            assert plan[2:] == want
+            assert plan[1] == "loom_hip_" + func + ("_f16" if want[2] == f16 else "")
+    assert accepted or base == f32
+
+
+@pytest.mark.parametrize("base", [bf, f16, f32])
+def test_prologue_plans(base):
+    shapes0 = [(1, 4, 128, 32), (1, 4, 128), (4,), (1, 2, 128, 64), (1, 2, 128, 64)]
+    accepted = 0
+    for (shapes, change), Q in itertools.product(_variants(shapes0), (64, 128, 48, 0, -64)):
+        types = [base, f32, f32, base, base]
+        if change:
+            types[change[0]] = change[1]
+        tensors = [_meta(t, s) for t, s in zip(types, shapes)]
+        sig = tuple(itertools.chain.from_iterable((t.dtype, t.shape) for t in tensors))
+        plan = lh._prologue_plan(sig, Q)
+        try:
+            lh.ssd_prologue(*tensors, Q)
+            want = "accepted"
+        except (ValueError, TypeError) as err:
+            want = str(err)
+        # the full checks accept the form, and stop at the device
+        assert (plan is not None) == ("ROCm device" in want), (shapes, types, Q, want)
+        if plan:
+            accepted += 1
+            b, H, L, P = shapes[0]
+            G, N = shapes[3][1], shapes[3][3]
+            assert plan[2] == (b, L // Q, H, G, Q, P, N)
+            assert [s for _, s in plan[3]] == [(b, H, L // Q, Q), (b, L // Q, G, Q, Q),
+                                               (b, L // Q, H, N, P)]
+    assert accepted or base == f32
+
+
+def test_cpu_calls_take_the_full_checks():
+    assert lh._enter("matmul", (torch.zeros(4, 4, dtype=bf), torch.zeros(4, 4, dtype=bf)), None,
+                     ()) is None
+    assert lh._enter("matmul", (None, 3), None, ()) is None
