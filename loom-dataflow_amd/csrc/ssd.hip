@@ -24,7 +24,8 @@
 //                      load issued before the first MFMA; the transposed
 //                      tile gives each lane four consecutive j of one row i
 //                      (8-byte stores).
-//   ssd_state_kernel   one workgroup per (b, h, 64-wide n block) walks the
+//   ssd_state_kernel   one workgroup per (b, h, 64-wide n block), and segment
+//                      of the sequence where those are few, walks its
 //                      chunks in order, keeping prev_states in the MFMA
 //                      accumulators: per chunk it stores prev(c), scales by
 //                      exp(dA[c,Q-1]) and accumulates states(c), so the
@@ -32,6 +33,8 @@
 //                      staged in LDS ([k][p], [k][n]) and read as MFMA
 //                      operands with ds_read_b64_tr_b16; w_c scales x in
 //                      fp32 and enters the MFMA as a bf16 hi + lo pair.
+//   ssd_carry_kernel   joins the segments: adds the decayed state at each
+//                      segment's start to the slots after it.
 #include "common.h"
 
 namespace {
@@ -199,6 +202,7 @@ struct SsdStateParams {
   int xbytes, bbytes;        // per stage
   int ninstr, lpw;           // DMA copies per unit; the most any wave issues
   int ns;                    // stages in the ring (3 .. 8; 2 in the WIDE form)
+  int cps;                   // chunks per segment (nc: one workgroup walks them all)
 };
 
 // MODE 0: tile t of wave w is w + 8 t, each with its own p tile.
@@ -230,7 +234,9 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
   const int n0 = nblk * nb;
   const int L = nc * Q;
   const int XR = P * 2, BR = nb * 2;
-  const int QS = WIDE ? 256 : p.QS, QSP = WIDE ? 256 : p.QSP, upc = p.upc, nu = nc * upc;
+  // this workgroup's chunks c0 .. c1 - 1, from a zero state
+  const int c0 = (int)blockIdx.z * p.cps, c1 = min(nc, c0 + p.cps);
+  const int QS = WIDE ? 256 : p.QS, QSP = WIDE ? 256 : p.QSP, upc = p.upc, nu = (c1 - c0) * upc;
   const int xbytes = WIDE ? QSP * P * 2 : p.xbytes, bbytes = WIDE ? QSP * nb * 2 : p.bbytes;
   const int stage_bytes = xbytes + bbytes + (WIDE ? 3072 : 2048);
   const int xinstr = xbytes / 1024, binstr = bbytes / 1024;
@@ -281,7 +287,7 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
   }
   // slots [i0, i1) of unit u
   auto issue = [&](int s, int u, int i0, int i1) {
-    const int c = u / upc, ko = (u % upc) * QS;
+    const int c = c0 + u / upc, ko = (u % upc) * QS;
     const int64_t key0 = (int64_t)c * Q + ko;   // first key of the unit within (b, h)
     const uint32_t base = lds_addr(sm + s * stage_bytes);
 #pragma unroll
@@ -301,7 +307,7 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
   // plus the lane's 32-bit byte offset (kept from the setup above: goff is
   // an element offset there).
   auto issue_wide = [&](int s, int u, int part) {
-    const int c = u / upc;
+    const int c = c0 + u / upc;
     const int64_t key0 = (int64_t)c * Q + (u % upc) * 256;
     const uint32_t base = lds_addr(sm + s * stage_bytes);
     if (part == 0) {
@@ -451,8 +457,39 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
     }
   };
 
+  // the running state to slot c of prev_states_T (MODE 2: the odd wave of a
+  // pair hands its partial sums to the even wave through LDS)
+  auto store_prev = [&](int c) {
+    float* outc = p.prevT + (((int64_t)(b * nc + c) * H + h) * N + n0) * P;
+    if constexpr (MODE == 2) {
+      const int pt = wave % ptiles;
+      f32x4_t* xch = s_x + pt * TPW * 64 + lane;
+      if (kq == 1) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) xch[t * 64] = R[t];
+      }
+      LOOM_WAIT_LGKM0();
+      barrier_nofence();
+      if (kq == 0) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+          *reinterpret_cast<f32x4_t*>(outc + (int64_t)(16 * t + r) * P + 16 * pt + 4 * gq) =
+              R[t] + xch[t * 64];
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        const int tt = wave + kSsdWaves * t;
+        if (tt < tiles) {
+          const int pt = tt % ptiles, nt = tt / ptiles;
+          *reinterpret_cast<f32x4_t*>(outc + (int64_t)(16 * nt + r) * P + 16 * pt + 4 * gq) = R[t];
+        }
+      }
+    }
+  };
+
   auto compute = [&](int s, int u) {
-    const int c = u / upc, part = u % upc;
+    const int c = c0 + u / upc, part = u % upc;
     const lds_char_t* xs = sm + s * stage_bytes;
     const lds_char_t* bs = xs + xbytes;
     const float* dAs = reinterpret_cast<const float*>(smem + s * stage_bytes + xbytes + bbytes);
@@ -464,37 +501,12 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
     make_w(dAs);
     lds_order();   // the w row's float stores before its f32x4 reads below
     if (part == 0) {
-      // prev(c) out, then R = exp(dA[c, Q-1]) R; states(c) accumulate below
+      // prev(c) out, then R = exp(dA[c, Q-1]) R; states(c) accumulate below.
+      // (A segment's first slot belongs to the segment before it.)
       const float decay = fast_exp2(dAs[2 * DTO + 3] * kLog2e);
-      float* outc = p.prevT + (((int64_t)(b * nc + c) * H + h) * N + n0) * P;
-      if constexpr (MODE == 2) {
-        const int pt = wave % ptiles;
-        f32x4_t* xch = s_x + pt * TPW * 64 + lane;
-        if (kq == 1) {
+      if (c > c0 || c0 == 0) store_prev(c);
 #pragma unroll
-          for (int t = 0; t < TPW; ++t) xch[t * 64] = R[t];
-        }
-        LOOM_WAIT_LGKM0();
-        barrier_nofence();
-        if (kq == 0) {
-#pragma unroll
-          for (int t = 0; t < TPW; ++t)
-            *reinterpret_cast<f32x4_t*>(outc + (int64_t)(16 * t + r) * P + 16 * pt + 4 * gq) =
-                R[t] + xch[t * 64];
-        }
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) R[t] *= decay;
-      } else {
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          const int tt = wave + kSsdWaves * t;
-          if (tt < tiles) {
-            const int pt = tt % ptiles, nt = tt / ptiles;
-            *reinterpret_cast<f32x4_t*>(outc + (int64_t)(16 * nt + r) * P + 16 * pt + 4 * gq) = R[t];
-            R[t] *= decay;
-          }
-        }
-      }
+      for (int t = 0; t < TPW; ++t) R[t] *= decay;
     }
     const int nks = QSP / 32;
     if constexpr (MODE >= 1) {
@@ -583,13 +595,81 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
     LOOM_WAIT_LGKM0();                        // this wave's reads of unit u-1's stage done
     barrier_nofence();
     compute(u % NS, u);
-    stores = (u % upc == 0) ? nst : 0;
+    stores = u % upc == 0 && (u > 0 || c0 == 0) ? nst : 0;
   }
+  if (c1 < nc) {               // the segment's own sum, to the next one's first slot
+    LOOM_WAIT_LGKM0();         // the last hand-over has been read
+    barrier_nofence();
+    store_prev(c1);
+  }
+}
+
+// Joins the segments of ssd_state_kernel.  Slot c of a segment that starts at
+// chunk c0 > 0 holds the state that the segment's own chunks give (slots c0 + 1
+// .. c0 + cps; slot c0 belongs to the segment before); what is missing is
+// prev(c0) times the decay since: w = prev(c0), then for every following slot
+// w *= exp(dA[c - 1, Q - 1]), prev(c) = slot + w, and at the next segment's
+// start w = prev(c).  One thread per four p of an (n, p) row of one (b, h); the
+// slots of a thread do not depend on each other, so eight loads are in flight.
+// Streams the slots after the first segment once, in and out.
+__global__ void __launch_bounds__(256) ssd_carry_kernel(const float* __restrict__ dA,
+                                                        float* prevT, int H, int nc, int Q,
+                                                        int NP4, int cps) {
+  const int e = (int)blockIdx.x * 256 + (int)threadIdx.x;
+  if (e >= NP4) return;
+  const int bh = blockIdx.y, b = bh / H, h = bh % H;
+  constexpr float kLog2e = 1.4426950408889634f;
+  const float* tail = dA + (int64_t)bh * nc * Q + Q - 1;     // dA[c, Q - 1] at c Q
+  f32x4_t* const base = reinterpret_cast<f32x4_t*>(prevT) + ((int64_t)b * nc * H + h) * NP4 + e;
+  const int64_t cs = (int64_t)H * NP4;                       // one chunk on
+  f32x4_t w = base[cps * cs];
+  constexpr int CH = 8;
+  int left = cps;                                            // slots until the next start
+  for (int ca = cps + 1; ca < nc; ca += CH) {
+    f32x4_t v[CH];
+    float d[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      const int c = min(ca + i, nc - 1);
+      v[i] = base[c * cs];
+      d[i] = tail[(int64_t)(c - 1) * Q];
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+      if (ca + i < nc) {
+        w *= fast_exp2(d[i] * kLog2e);
+        const f32x4_t t = v[i] + w;
+        base[(ca + i) * cs] = t;
+        if (--left == 0) {
+          w = t;
+          left = cps;
+        }
+      }
+    }
+  }
+}
+
+// Chunks per segment of the state kernel.  Its workgroups, one per (b, h,
+// n block), walk a sequence's chunks one after the other, about (Q + 50) / 150
+// us each; where they are at most half the CUs, the sequence is cut into as
+// many segments as give about one workgroup per CU, if what that saves is more
+// than joining them costs (ssd_carry_kernel: about 3 us and the later slots in
+// and out at 4 TB/s).  Whole prologue, L 4096: b1 H32 P64 N128 Q256 (64
+// workgroups, 4 segments) 41.2 -> 25.8 us, H8 39.1 -> 16.6, b2 43.3 -> 36.4; H8
+// P32 N64 Q256 L 8192 128 -> 21; with b4's 256 workgroups 49.9, and 62.5 cut in
+// two.
+int segment_chunks(const SsdStateParams& p, int64_t workgroups, int64_t state_floats, int cus) {
+  const int nseg = (int)std::min<int64_t>(p.nc, cus / workgroups);
+  if (nseg < 2) return p.nc;
+  const int cps = (p.nc + nseg - 1) / nseg;
+  const int64_t later = p.nc - cps, saved = later * (p.Q + 50);       // in 1/150 us
+  return saved > 450 + later * state_floats * 8 / 26667 ? cps : p.nc;
 }
 
 template <int TPW, bool F16>
 void launch_state(const SsdStateParams& p, int mode, int grid_x, int grid_y, hipStream_t st) {
-  const dim3 grid((unsigned)grid_x, (unsigned)grid_y), block(64 * kSsdWaves);
+  const dim3 grid((unsigned)grid_x, (unsigned)grid_y, (unsigned)((p.nc + p.cps - 1) / p.cps));
+  const dim3 block(64 * kSsdWaves);
   if constexpr (TPW == 4) {
     if (mode == 2 && p.QS == 256) {
       hipLaunchKernelGGL((ssd_state_kernel<4, 2, F16, true>), grid, block, 0, st, p);
@@ -768,10 +848,16 @@ int state_passing_impl(const void* x, const void* dt, const void* dA_cumsum,
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int gx = (int)(batch * nheads), gy = (int)(dstate / nb);
   if (loom_validate_only()) return loom_ok(err, errlen);
+  p.cps = segment_chunks(p, (int64_t)gx * gy, (int64_t)gx * p.N * p.P, stream_cus(st));
   if (tpw <= 1) launch_state<1, F16>(p, mode, gx, gy, st);
   else if (tpw <= 2) launch_state<2, F16>(p, mode, gx, gy, st);
   else launch_state<4, F16>(p, mode, gx, gy, st);
-  return loom_check_launch(err, errlen, "ssd_chunk_state_passing");
+  rc = loom_check_launch(err, errlen, "ssd_chunk_state_passing");
+  if (rc || p.cps == p.nc) return rc;
+  const int np4 = p.N * p.P / 4;
+  hipLaunchKernelGGL(ssd_carry_kernel, dim3((unsigned)((np4 + 255) / 256), (unsigned)gx), dim3(256),
+                     0, st, p.dA, p.prevT, p.H, p.nc, p.Q, np4, p.cps);
+  return loom_check_launch(err, errlen, "ssd_chunk_state_passing (segments)");
 }
 
 template <bool F16>
