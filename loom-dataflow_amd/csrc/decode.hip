@@ -869,14 +869,15 @@ int flash_decode_impl(const void* k, const void* v, const void* q, void* out,
   }
   int rc = loom_check_launch(err, errlen, "flash_decode (split)");
   if (rc) return rc;
-  // Few splits, one thread per two d of a row; many, one workgroup per row.
-  // At 9 to 16 splits the former while its threads cover the CUs (B32 H32 D128
-  // S8192 in 16 splits: 32.7 against 33.5 us), the latter for fewer rows (B4
-  // H32 S1025 in 17: 10.3 -> 8.7)
+  // Up to 16 splits, one thread per two d of a row; more, one workgroup per
+  // row.  At 16 splits the two take the same time for few rows (B4 H32 D128
+  // S1024: 8.2 us both) and the former less for many (B32 H32 D128 S8192 32.7
+  // against 33.5 us, B22 H48 D64 S9168 in 12 19.3 against 20.6); at 17 the
+  // former needs a second round trip
   const dim3 cgrid((unsigned)cdiv64(B * H * D / 2, 256)), cblock(256);
   if (p.ns <= 8)
     hipLaunchKernelGGL((decode_combine_kernel<F16, 8>), cgrid, cblock, 0, st, p);
-  else if (p.ns <= 16 && (int64_t)cgrid.x >= 256)
+  else if (p.ns <= 16)
     hipLaunchKernelGGL((decode_combine_kernel<F16, 16>), cgrid, cblock, 0, st, p);
   else
     hipLaunchKernelGGL((decode_combine_row_kernel<F16>), dim3((unsigned)(B * H)), cblock, 0, st, p);
