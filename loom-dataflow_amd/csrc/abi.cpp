@@ -793,29 +793,36 @@ int loom_hip_preferred_block_sizes(const char* func, const int64_t* dims, int nd
   // a workgroup tile T bound within natural_ub: T itself, or the whole
   // extent when that is below T (it runs as T)
   auto bound = [](long long T, long long extent) { return std::min(T, extent); };
-  // largest square GEMM tile that still gives every CU a workgroup, among
-  // those a binding can name for these extents
-  auto gemm_pick = [&](long long M, long long N, long long z) {
+  // Square GEMM tile, among those a binding can name for these extents.  The
+  // 64 tile while two of its workgroups per CU hold the product in one round
+  // and 128 would not give every CU one (1280x1280x2048: 19.2 against 19.5 us;
+  // past that line 7872x384x6016 87 against 66, 1536^3 20.4 against 15.6).  The
+  // 256 tile where the contraction is long enough to pay for its epilogue and
+  // it gives every CU a workgroup, or 128 would take a second round (3000^3,
+  // 144 tiles of 256 against 576 of 128: 65 against 89 us; 2560x2560x4096, 100
+  // against 400: 71 against 67; K 96, 2688x6912: 23 against 16).
+  auto gemm_pick = [&](long long M, long long N, long long z, long long K) {
     auto nameable = [&](long long T, long long E) {
       return T <= E || (T == 64 && E < 64) || (T == 128 && E > 64 && E < 128) ||
              (T == 256 && E > 128 && E < 256);
     };
-    for (long long t : {256LL, 128LL})
-      if (nameable(t, M) && nameable(t, N) && ceil_div(M, t) * ceil_div(N, t) * z >= kCUs) {
-        b["tile_m"] = bound(t, M);
-        b["tile_n"] = bound(t, N);
-        return;
-      }
-    // 64 is nameable on every axis (64 itself, or an extent below it)
-    b["tile_m"] = bound(64, M);
-    b["tile_n"] = bound(64, N);
+    auto tiles = [&](long long T) { return ceil_div(M, T) * ceil_div(N, T) * z; };
+    long long t = 64;   // nameable on every axis (64 itself, or an extent below it)
+    if (nameable(256, M) && nameable(256, N) && K >= 512 &&
+        (tiles(256) >= kCUs || (K >= 768 && tiles(128) > 2 * kCUs)))
+      t = 256;
+    else if (nameable(128, M) && nameable(128, N) &&
+             (tiles(128) >= kCUs || tiles(64) > 2 * kCUs))
+      t = 128;
+    b["tile_m"] = bound(t, M);
+    b["tile_n"] = bound(t, N);
   };
   if (f == "matmul") {
-    gemm_pick(d[0], d[1], 1);
+    gemm_pick(d[0], d[1], 1, d[2]);
     b["tile_k"] = std::min<long long>(64, d[2]);
   } else if (f == "batch_matmul") {
     b["tile_b"] = 1;
-    gemm_pick(d[1], d[2], d[0]);
+    gemm_pick(d[1], d[2], d[0], d[3]);
     b["tile_k"] = std::min<long long>(64, d[3]);
   } else if (f == "split_k_matmul_gather") {
     // 128x128 tiles (64x64 when M or N is small), enough K slabs to cover

@@ -374,13 +374,55 @@ def _run(plan, *args):
 # kernels (examples/<k>/IR/00_from_helion_frontend.mlir)
 # ---------------------------------------------------------------------------
 
+@functools.lru_cache(maxsize=1024)
+def _slabs(M, N, K):
+    """K slab of a matmul whose tiles the library chooses, or 0 for one pass.
+
+    A product of few 64 x 64 tiles leaves CUs idle, each of the others
+    pulling its panels at about 60 KB/us whatever is in flight: with at most
+    one tile per two CUs (of 256) and a long K, slabs that give about one
+    workgroup per CU are multiplied side by side (split_k_matmul_gather's
+    kernels: fp32 partials, added in ascending order).  The second launch and
+    the partials cost about 3.5 us on the GPU and 5 on the host, so the line
+    lies where one pass takes longer than the host's way to two: 40x576x8064
+    22.9 -> 8.7 us, 1216x128x7488 26.9 -> 12.8, 16x4096x4096 14.2 -> 11.4, and
+    with rows off 16-byte boundaries 56x775x6976 44.2 -> 12.2; but 128x128x1024
+    5.8 against 6.8."""
+    t = -(-M // 64) * -(-N // 64)
+    s = min(16, 256 // t, K // 256)
+    if s < 2:
+        return 0
+    tk = -(-(-(-K // s)) // 64) * 64
+    least, saved = (3200, 1400) if K % 8 == 0 and N % 8 == 0 else (1700, 800)
+    return tk if K >= least and K - tk >= saved else 0
+
+
+def _matmul_slabs(plan, x, y, out, tk, st) -> bool:
+    """The product in K slabs of tk; False where there is no memory for the
+    partials (at most 4 MB)."""
+    M, N, K = plan[2]
+    try:
+        partials = torch.empty((-(-K // tk), M, N), dtype=_fp32, device=x.device)
+    except torch.OutOfMemoryError:
+        return False
+    name = "loom_hip_split_k_matmul_gather" + ("_f16" if plan[4] == _f16 else "")
+    _run((getattr(_lib, name), name), x.data_ptr(), y.data_ptr(), out.data_ptr(),
+         partials.data_ptr(), partials.numel() * 4, M, N, K, plan[3][0], plan[3][1], tk, st)
+    return True
+
+
 def matmul(x, y, out=None, *, tile_m=None, tile_n=None, tile_k=None):
     """@matmul (examples/mm/IR/00_from_helion_frontend.mlir:2): out = x . y.
-    Tiles left as None take the preferred binding for the extents."""
+    Tiles left as None take the preferred binding for the extents; with all
+    three left so, a long K over few tiles is summed in slabs (_slabs)."""
     go = _enter("matmul", (x, y), out,
                 (("tile_m", tile_m), ("tile_n", tile_n), ("tile_k", tile_k)))
     if go:
         plan, out, st = go
+        if tile_m is None and tile_n is None and tile_k is None:
+            tk = _slabs(*plan[2])
+            if tk and _matmul_slabs(plan, x, y, out, tk, st):
+                return out
         _run(plan, x.data_ptr(), y.data_ptr(), out.data_ptr(), *plan[2], *plan[3], st)
         return out
     e, sfx = _elt(x)
