@@ -218,7 +218,10 @@ struct SsdStateParams {
 // WIDE (MODE 2, TPW 4, QS = 256): the unit layout and every wave's DMA
 //         slots are compile-time constants; one wait, barrier, w_c build and
 //         prev hand-over per 256 keys instead of two.
-template <int TPW, int MODE, bool F16, bool WIDE = false>
+// SEG: the grid's z walks segments of the sequence; without it the bounds are
+//         constants (b3 H24 L 1920 P128 N64 Q128, unsegmented: 65.5 us against
+//         68.2 with the bounds taken at run time).
+template <int TPW, int MODE, bool F16, bool SEG, bool WIDE = false>
 __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParams p) {
   static_assert(!WIDE || (MODE == 2 && TPW == 4), "256-key units: P = 64, nb = 64 only");
   __shared__ __attribute__((aligned(1024))) char smem[kSsdRing];
@@ -235,7 +238,7 @@ __global__ void __launch_bounds__(64 * kSsdWaves) ssd_state_kernel(SsdStateParam
   const int L = nc * Q;
   const int XR = P * 2, BR = nb * 2;
   // this workgroup's chunks c0 .. c1 - 1, from a zero state
-  const int c0 = (int)blockIdx.z * p.cps, c1 = min(nc, c0 + p.cps);
+  const int c0 = SEG ? (int)blockIdx.z * p.cps : 0, c1 = SEG ? min(nc, c0 + p.cps) : nc;
   const int QS = WIDE ? 256 : p.QS, QSP = WIDE ? 256 : p.QSP, upc = p.upc, nu = (c1 - c0) * upc;
   const int xbytes = WIDE ? QSP * P * 2 : p.xbytes, bbytes = WIDE ? QSP * nb * 2 : p.bbytes;
   const int stage_bytes = xbytes + bbytes + (WIDE ? 3072 : 2048);
@@ -666,22 +669,28 @@ int segment_chunks(const SsdStateParams& p, int64_t workgroups, int64_t state_fl
   return saved > 450 + later * state_floats * 8 / 26667 ? cps : p.nc;
 }
 
-template <int TPW, bool F16>
-void launch_state(const SsdStateParams& p, int mode, int grid_x, int grid_y, hipStream_t st) {
+template <int TPW, bool F16, bool SEG>
+void launch_state_impl(const SsdStateParams& p, int mode, int grid_x, int grid_y, hipStream_t st) {
   const dim3 grid((unsigned)grid_x, (unsigned)grid_y, (unsigned)((p.nc + p.cps - 1) / p.cps));
   const dim3 block(64 * kSsdWaves);
   if constexpr (TPW == 4) {
     if (mode == 2 && p.QS == 256) {
-      hipLaunchKernelGGL((ssd_state_kernel<4, 2, F16, true>), grid, block, 0, st, p);
+      hipLaunchKernelGGL((ssd_state_kernel<4, 2, F16, SEG, true>), grid, block, 0, st, p);
       return;
     }
   }
   if (mode == 2)
-    hipLaunchKernelGGL((ssd_state_kernel<TPW, 2, F16>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((ssd_state_kernel<TPW, 2, F16, SEG>), grid, block, 0, st, p);
   else if (mode == 1)
-    hipLaunchKernelGGL((ssd_state_kernel<TPW, 1, F16>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((ssd_state_kernel<TPW, 1, F16, SEG>), grid, block, 0, st, p);
   else
-    hipLaunchKernelGGL((ssd_state_kernel<TPW, 0, F16>), grid, block, 0, st, p);
+    hipLaunchKernelGGL((ssd_state_kernel<TPW, 0, F16, SEG>), grid, block, 0, st, p);
+}
+
+template <int TPW, bool F16>
+void launch_state(const SsdStateParams& p, int mode, int grid_x, int grid_y, hipStream_t st) {
+  if (p.cps < p.nc) launch_state_impl<TPW, F16, true>(p, mode, grid_x, grid_y, st);
+  else launch_state_impl<TPW, F16, false>(p, mode, grid_x, grid_y, st);
 }
 
 int check_ssd(const char* fn, int64_t batch, int64_t nchunks, int64_t nheads, int64_t ngroups,
