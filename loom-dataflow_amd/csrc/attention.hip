@@ -50,7 +50,8 @@ struct AttnParams {
 // W / KG waves of 16 QT query rows share each K/V stage.  KG 2: two waves
 // share a query tile, each taking one 32-key half of every stage, and merge at
 // the end: half the steps in a row's chain, for grids with few workgroups.
-// NSX: stages when nonzero; WPE: waves per SIMD the registers must allow.
+// NSX: stages when nonzero; WPE: waves per SIMD the registers must allow; DC:
+// the head dim that is computed, for narrower heads in the stages of D.
 // Softmax rescaling is
 // lazy: a row's running max only moves (and O, l are rescaled) when a block
 // raises it by more than 8 in the log2 domain, which keeps P <= 2^8 and the
@@ -87,7 +88,7 @@ LOOM_DEV int q_swz(int lr) { return D >= 128 ? (lr & 15) : ((lr ^ (lr >> 3)) & 7
 // piece reaches past its row), issued before the block NS-1 stages ahead of
 // the one being computed and written to the same LDS position after that
 // computation; V keeps its DMA.
-template <int D, int QT, int W, bool H, bool KREG, int KG = 1, int NSX = 0, int WPE = 1>
+template <int D, int QT, int W, bool H, bool KREG, int KG = 1, int NSX = 0, int WPE = 1, int DC = D>
 __global__ void __launch_bounds__(64 * W, WPE) attention_dma_kernel(AttnParams p) {
   constexpr int KB = 64;                        // keys per stage
   static_assert(KG == 1 || KG == 2, "a stage has two 32-key halves");
@@ -103,7 +104,7 @@ __global__ void __launch_bounds__(64 * W, WPE) attention_dma_kernel(AttnParams p
   constexpr int LPW = K_INSTR + V_INSTR;
   constexpr int VROW = D * 2;                   // Vs row bytes
   constexpr int V_ROWS_PER_I = 1024 / VROW;
-  constexpr int DSTEPS = D / 32, DT = D / 16;
+  constexpr int DSTEPS = DC / 32, DT = DC / 16;
   static_assert(LPW * (NS - 2) <= 63, "vmcnt range");
   // Q reaches LDS by DMA up to D 128 (a region after the stages, which also
   // stages O for the epilogue); at D 256 the two 64 KB stages leave no room
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(64 * W, WPE) attention_dma_kernel(AttnParams p
   // block) and writes them back as whole rows, 16 bytes per lane: 8-byte
   // stores of 32-byte row pieces cost the workgroup's end far more.
   if constexpr (QDMA) {
-    if (Dr == D) {
+    if (DC == D && Dr == D) {
 #pragma unroll
       for (int qt = 0; qt < QT; ++qt) {
         const float inv = 1.f / lacc[qt][0];
@@ -569,7 +570,14 @@ void launch_attention(AttnParams p, int64_t D, int64_t tile_m, hipStream_t st) {
   // four waves and three stages and 53 with four waves and two); at D 64
   // and more than two workgroups per CU four waves, of which four fit (BH128
   // S512 causal 10.9 against 13.4 us, but BH32 S333 x 1003 15.2 against 12.0)
-  switch ((D == 128 ? 10 : 0) + (int)(tile_m / 64)) {
+  // Heads of up to 96 in the stages of 128 skip the MFMAs of the last 32: BH128
+  // S3456 D96 causal 455 -> 403 us, BH128 2728 x 1754 D96 348 -> 306, BH96 S1024
+  // D72 65 -> 55
+  switch ((D == 128 ? p.D <= 96 ? 20 : 10 : 0) + (int)(tile_m / 64)) {
+    case 21: launch(attention_dma_kernel<128, 1, 8, H, KREG, 2, 2, 2, 96>, b8); break;
+    case 22: launch(attention_dma_kernel<128, 1, 8, H, KREG, 1, 0, 1, 96>, b8); break;
+    case 23: launch(attention_dma_kernel<128, 3, 4, H, KREG, 1, 0, 1, 96>, b4); break;
+    case 24: launch(attention_dma_kernel<128, 2, 8, H, KREG, 1, 0, 1, 96>, b8); break;
     case 11: launch(attention_dma_kernel<128, 1, 8, H, KREG, 2, 2, 2>, b8); break;
     case 12: launch(attention_dma_kernel<128, 1, 8, H, KREG>, b8); break;
     case 13: launch(attention_dma_kernel<128, 3, 4, H, KREG>, b4); break;

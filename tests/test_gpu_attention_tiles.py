@@ -89,3 +89,13 @@ def test_nan_reaches_the_row(lh):
         kt = dev(k)
         kt[0, 3, key] = float("nan")
         assert torch.isnan(lh.attention(kt, dev(v), dev(q))).all(), key
+
+
+# head dims whose products run over 96 of the 128 staged columns, at each query
+# tile, and 104 beside them; V rows of odd pieces (61 keys) take K by registers
+@pytest.mark.parametrize("D,tile_m", [(80, 64), (96, 64), (96, 128), (80, 192), (88, 256),
+                                      (96, 256), (104, 256)])
+@pytest.mark.parametrize("BH,Sq,Skv,causal", [(216, 270, 270, True), (216, 257, 61, False),
+                                              (24, 130, 130, True)])
+def test_heads_of_up_to_96(lh, D, tile_m, BH, Sq, Skv, causal):
+    _check(lh, BH, Sq, Skv, D, causal, min(tile_m, Sq), (0, BH // 2, BH - 1))
