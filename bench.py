@@ -375,7 +375,7 @@ def make_cases(torch, lh):
         return dict(fn=lambda i: lh.matmul(*sets[i % n], tile_m=64, tile_n=64, tile_k=64),
                     flop=2 * 1024 ** 3, bytes=3 * 1024 * 1024 * 2, bound="mfma", sets=n,
                     iters=max(n, 20), desc=f"mm 1024^3 bf16, tile 64x64 ({what})", cpu=cpu,
-                    kernel="gemm_pipe_kernel<64, false, false>")
+                    kernel="gemm_pipe_kernel<64, false, false, true>")
     cases["mm"] = lambda: mm_case(160, "operands from HBM: 160 rotating copies")
     cases["mm_warm"] = lambda: mm_case(1, "operands cache resident")
 
@@ -414,7 +414,7 @@ def make_cases(torch, lh):
                                                           tile_k=1024),
                     flop=2 * 512 * 512 * 16384, bytes=nb, bound="hbm", sets=n,
                     desc="split-K 512x512x16384, 16 slabs, fp32 partials", cpu=cpu,
-                    kernel="gemm_pipe_kernel<128, true, false>")
+                    kernel="gemm_pipe_kernel<128, true, false, true>")
     cases["split_k"] = splitk
 
     def flashattn():
@@ -431,7 +431,7 @@ def make_cases(torch, lh):
         return dict(fn=lambda i: lh.attention(*sets[i % n], causal=True, tile_m=256, tile_n=64),
                     flop=4 * BH * S * S * D // 2, bytes=nb, bound="mfma", sets=n,
                     desc="flashattn fwd B4 H32 S4096 D128 causal, tile_m 256", cpu=cpu,
-                    kernel="attention_dma_kernel<128, 2, 8, false, false>")
+                    kernel="attention_dma_kernel<128, 2, 8, false, false, 1, 0, 1, 128>")
     cases["flashattn"] = flashattn
 
     def decode():
@@ -518,7 +518,7 @@ def make_cases(torch, lh):
             return 1 / b, "batch 1 of 4", lambda: oracle.mamba_prologue(*a, Q)
         return dict(fn=fn, out=out, flop=flop, bytes=nb, bound="hbm", sets=n,
                     desc="mamba SSD prologue (cumsum, cb, states + passing) b4 L4096 h32 P64 "
-                         "N128 g1 Q256", cpu=cpu, kernel="ssd_state_kernel<4, 2, false, true>")
+                         "N128 g1 Q256", cpu=cpu, kernel="ssd_state_kernel<4, 2, false, false, true>")
     cases["mamba_prologue"] = ssd
     return cases
 

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import oracle
+from tests.test_gpu_graph import _replay_matches
 from tests.test_gpu_parity import dev, host
 from tests.test_gpu_random_shapes import _ints
 
@@ -34,6 +35,16 @@ def test_matmul_slabs(lh, M, N, K):
     assert torch.equal(got, one)
     out = torch.empty_like(got)
     assert lh.matmul(dev(x), dev(y), out) is out and torch.equal(out, got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 576, 4096), (33, 47, 1700)])
+def test_slabs_captured(lh, M, N, K):
+    """The partials' allocation and both launches inside a graph."""
+    rng = np.random.default_rng(M)
+    x, y = dev(_ints(rng, (M, K))), dev(_ints(rng, (K, N)))
+    out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    _replay_matches(f"matmul slabs {M}x{N}x{K}", lambda: lh.matmul(x, y, out), [out])
 
 
 def test_rule():

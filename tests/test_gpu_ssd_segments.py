@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from tests.test_gpu_graph import _replay_matches
 from tests.test_gpu_ssd import _check_prologue, _raw_inputs
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,16 @@ def test_segments(lh, P, N, Q, b, H, nc):
     x, dt, A, Bm, C = _raw_inputs(rng, b, H, 1, nc * Q, P, N, dt_scale=0.01)
     print(f"segments b{b} H{H} nc{nc} Q{Q} P{P} N{N}", flush=True)
     _check_prologue(lh, x, dt, A, Bm, C, Q, f"b{b} H{H} nc{nc} Q{Q} P{P} N{N}")
+
+
+def test_segments_captured(lh):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    b, H, nc, Q, P, N = 1, 4, 16, 256, 64, 128
+    L = nc * Q
+    x = torch.randn(b, H, L, P, device="cuda", generator=g).to(torch.bfloat16)
+    dt = torch.rand(b, H, L, device="cuda", generator=g) * 0.01
+    A = -torch.rand(H, device="cuda", generator=g)
+    Bm, C = (torch.randn(b, 1, L, N, device="cuda", generator=g).to(torch.bfloat16) for _ in "BC")
+    _, dA, cb, prev = lh.ssd_prologue(x, dt, A, Bm, C, Q)
+    _replay_matches("ssd segments", lambda: lh.ssd_prologue(
+        x, dt, A, Bm, C, Q, dA_cumsum=dA, cb=cb, prev_states_T=prev), [dA, cb, prev])
