@@ -350,6 +350,12 @@ def _enter(func: str, tensors, out, given: tuple):
                 return None
             sig.append(t.dtype)
             sig.append(t.shape)
+        # a tile may be any object with an integer value (a tensor is hashed by
+        # identity, and its value can change): the key holds the value
+        for _, v in given:
+            if v is not None and type(v) is not int:
+                given = tuple((s, v if v is None else int(v)) for s, v in given)
+                break
         plan = _plan(func, tuple(sig), given) if i >= 0 else None
         if plan is None:
             return None
@@ -358,7 +364,7 @@ def _enter(func: str, tensors, out, given: tuple):
         elif not isinstance(out, torch.Tensor) or out.dtype != plan[4] or \
                 tuple(out.shape) != plan[5] or out.get_device() != i or not out.is_contiguous():
             return None
-    except (AttributeError, TypeError, RuntimeError):
+    except (AttributeError, TypeError, ValueError, OverflowError, RuntimeError):
         return None
     return plan, out, _raw_stream(i)
 

@@ -2,7 +2,9 @@
 exactly the signatures that the full checks accept, and gives the same
 extents, tiles and output shapes (CPU only: signatures are types and shapes)."""
 import itertools
+import weakref
 
+import numpy as np
 import pytest
 import torch
 
@@ -105,6 +107,39 @@ def test_prologue_plans(base):
             assert [s for _, s in plan[3]] == [(b, H, L // Q, Q), (b, L // Q, G, Q, Q),
                                                (b, L // Q, H, N, P)]
     assert accepted or base == f32
+
+
+class _OnDevice(torch.Tensor):
+    """A tensor without memory that says it lies on device 0, as _enter asks."""
+
+    def get_device(self):
+        return 0
+
+
+def _on_device(dtype, shape):
+    return _meta(dtype, shape).as_subclass(_OnDevice)
+
+
+def test_plans_hold_the_value_of_a_tile(monkeypatch):
+    """A tile given as an object whose value changes: each call takes the value
+    it has then, and the plan keeps no reference to the object."""
+    monkeypatch.setattr(lh, "_raw_stream", lambda i: 0)
+    ab = _on_device(bf, (64, 512)), _on_device(bf, (512, 48))
+
+    def tiles(tk):
+        return lh._enter("split_k_matmul_gather", ab, None,
+                         (("tile_m", 64), ("tile_n", None), ("tile_k", tk)))[0][3]
+    tk = torch.tensor(128)
+    assert tiles(tk) == (64, 48, 128)
+    tk.fill_(256)
+    assert tiles(tk) == (64, 48, 256)
+    dead = weakref.ref(tk)
+    del tk
+    assert dead() is None
+    for value in (np.int64(64), 64.0, 64):
+        assert tiles(value) == (64, 48, 64)
+    for value in (float("inf"), float("nan"), "x", (1,)):     # the full checks say what is wrong
+        assert lh._enter("matmul", ab, None, (("tile_m", value),)) is None
 
 
 def test_cpu_calls_take_the_full_checks():
