@@ -644,7 +644,7 @@ def _prologue_plan(sig: tuple, Q):
     prologue's signature (x, dt, A, B, C), or None; see _plan."""
     dtypes, (xs, dts, As, Bs, Cs) = sig[0::2], [tuple(v) for v in sig[1::2]]
     e = dtypes[0]
-    if len(xs) != 4 or len(Bs) != 4 or e not in (_bf16, _f16) or not isinstance(Q, int):
+    if len(xs) != 4 or len(Bs) != 4 or e not in (_bf16, _f16):
         return None
     (b, H, L, P), G, N = xs, Bs[1], Bs[3]
     if Q <= 0 or L % Q or dtypes != (e, _fp32, _fp32, e, e) or dts != (b, H, L) or As != (H,) or \
@@ -660,6 +660,8 @@ def _enter_prologue(ins, outs, Q):
     """(plan, outputs, stream) of a well-formed prologue call, or None."""
     try:
         i = ins[0].get_device()
+        if type(Q) is not int:    # other types' keys could compare equal to an int's
+            return None
         sig = []
         for t in ins:
             if not isinstance(t, torch.Tensor) or t.get_device() != i or not t.is_contiguous():

@@ -142,6 +142,17 @@ def test_plans_hold_the_value_of_a_tile(monkeypatch):
         assert lh._enter("matmul", ab, None, (("tile_m", value),)) is None
 
 
+def test_prologue_chunk_size_of_another_type(monkeypatch):
+    """A chunk size that is no int goes the full way and leaves the int's own
+    plan alone, though the two compare and hash equal."""
+    monkeypatch.setattr(lh, "_raw_stream", lambda i: 0)
+    ins = [_on_device(t, s) for t, s in zip(
+        (bf, f32, f32, bf, bf), [(1, 4, 96, 32), (1, 4, 96), (4,), (1, 2, 96, 64), (1, 2, 96, 64)])]
+    for Q in (np.int64(48), 48.0, torch.tensor(48)):
+        assert lh._enter_prologue(ins, (None,) * 3, Q) is None
+    assert lh._enter_prologue(ins, (None,) * 3, 48)[0][2] == (1, 2, 4, 2, 48, 32, 64)
+
+
 def test_cpu_calls_take_the_full_checks():
     assert lh._enter("matmul", (torch.zeros(4, 4, dtype=bf), torch.zeros(4, 4, dtype=bf)), None,
                      ()) is None
