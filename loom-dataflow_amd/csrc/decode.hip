@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(64 * W) decode_dma_kernel(DecodeParams p) {
         st[j][i] = v;
       }
     // ---- lazy online softmax: the base moves (and O, l rescale) only on
-    // this wave's first block or when a score rises more than 8 above it
+    // this wave's first blocks or when a score rises more than 8 above it
     float mx = -INFINITY;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -380,17 +380,18 @@ __global__ void __launch_bounds__(64 * W) decode_dma_kernel(DecodeParams p) {
       // masking is per key, so a block is masked for every head or for none:
       // a wholly masked first block adds nothing and leaves the base unset
       if (first && __builtin_amdgcn_ballot_w64(mx != -INFINITY) == 0) return;
-      const float shift = first ? mx : fmaxf(mx, 0.f);
-      if (!first) {
-        const float alpha = fast_exp2(-shift);
-        lacc *= alpha;
+      // scores of -inf are per head: a head's base is set by its first block
+      // with a finite one, until which its l is zero
+      const bool unset = first && lacc[0] == 0.f;
+      const float shift = unset ? (mx == -INFINITY ? 0.f : mx) : fmaxf(mx, 0.f);
+      const float alpha = unset ? 1.f : fast_exp2(-shift);
+      lacc *= alpha;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) ot[dt] *= alpha;
-      }
+      for (int dt = 0; dt < DT; ++dt) ot[dt] *= alpha;
       m_run += shift;
 #pragma unroll
       for (int j = 0; j < 2; ++j) st[j] -= shift;
-      first = false;
+      first = __builtin_amdgcn_ballot_w64(unset && mx == -INFINITY) != 0;
     }
     f32x4_t e0, e1;
 #pragma unroll
