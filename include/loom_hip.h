@@ -110,9 +110,9 @@ int loom_hip_split_k_matmul_gather(const void* a, const void* b, void* out, void
  * reference hard-codes the f16 constant 0.08837890625 at :10); `causal`
  * (not in the reference; needs Sq == Skv) hides key j from query i < j.
  * tile_m (a multiple of 16 up to Sq, or Sq) runs as the smallest workgroup
- * query tile of 64, 128, 192, 256 covering it, or as 64 rows where that tile
- * would leave CUs idle (the 64-row tile sums a row's keys in two halves, so its
- * results differ from the others' in rounding); tile_b (<= BH) and tile_n (<= Skv, the
+ * query tile of 64, 128, 192, 256 covering it (the 64-row tile may sum a row's
+ * keys in two halves, so its results can differ from the others' in rounding);
+ * tile_b (<= BH) and tile_n (<= Skv, the
  * online-softmax step) are validated, the kernel streams KV in 64-key LDS
  * blocks.  D a multiple of 8 up to 256 (built for 64, 128 and 256; a
  * narrower D runs on the next one up with its padding rows zero; above 128
@@ -478,7 +478,10 @@ int loom_hip_hw_spec(int device, char* out, size_t outlen, char* err, size_t err
 
 /* The binding this library runs fastest for those extents on MI355X (one
  * JSON object {"tile_m": 256, ...} over the function's symbols; a legal
- * point of loom_hip_constraint_scope), usable as a block_sizes_json entry. */
+ * point of loom_hip_constraint_scope), usable as a block_sizes_json entry.
+ * The extents of attention do not say whether a call is causal: its tile_m is
+ * that of a call that is not, and a causal one up to D 128 with between 512
+ * and 1024 workgroups of 64 rows runs faster on 64. */
 int loom_hip_preferred_block_sizes(const char* func, const int64_t* dims, int ndims, char* out,
                                    size_t outlen, char* err, size_t errlen);
 

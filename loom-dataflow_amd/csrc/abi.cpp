@@ -838,10 +838,23 @@ int loom_hip_preferred_block_sizes(const char* func, const int64_t* dims, int nd
     b["tile_k"] = std::min<long long>(d[2], ceil_div(ceil_div(d[2], S), step) * step);
   } else if (f == "attention") {
     b["tile_b"] = 1;
-    // 256 query rows (128 for head dims above 128), or the largest built
-    // tile within a shorter Sq (Sq itself below 64)
+    // 64 query rows where a larger tile would leave CUs idle or uneven; else 256
+    // (128 for head dims above 128), or the largest built tile within a
+    // shorter Sq (Sq itself below 64).  The large tiles read each K/V stage
+    // once for up to four times the rows, but a workgroup of 256 rows takes
+    // about 1.9 us per 64-key block (one fits a CU) where 64 rows take 0.65,
+    // two workgroups to a CU: the line lies where their rounds cost the same,
+    // at two workgroups of 64 rows per CU (BH32 D128 not causal, S1000, two per
+    // CU: 26 us against 33; S2048, four per CU: 86 against 67).  A causal
+    // grid's line is at four (loom_hip's Python calls take it there: S1000 19
+    // against 33, S2048 49 against 61, but BH128 S1024, eight per CU, 56
+    // against 50).  Above D 128 the large tile is 128 rows and the line at one
+    // workgroup per CU (BH8 S1000 causal 27 against 39).
     const long long top = d[3] > 128 ? 128 : 256;
-    b["tile_m"] = d[1] >= top ? top : d[1] >= 192 ? 192 : d[1] >= 128 ? 128 : d[1] >= 64 ? 64 : d[1];
+    if (d[0] * ceil_div(d[1], 64) <= (d[3] > 128 ? 1 : 2) * kCUs)
+      b["tile_m"] = bound(64, d[1]);
+    else
+      b["tile_m"] = d[1] >= top ? top : d[1] >= 192 ? 192 : d[1] >= 128 ? 128 : bound(64, d[1]);
     b["tile_n"] = std::min<long long>(64, d[2]);
   } else if (f == "flash_decode") {
     b["tile_b"] = 1;

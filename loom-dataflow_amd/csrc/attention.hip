@@ -538,25 +538,8 @@ __global__ void __launch_bounds__(64 * W, WPE) attention_dma_kernel(AttnParams p
   }
 }
 
-// The workgroup query tile a binding's tile (64 .. 256) runs on: 64 rows where
-// the larger tile would leave CUs idle or uneven, else the binding's own.
-// The large tiles read each K/V stage once for up to four times the rows, but
-// a workgroup of 256 rows takes about 1.9 us per 64-key block (one fits a CU)
-// where 64 rows take 0.65, two workgroups to a CU: the line lies where their
-// rounds cost the same, at two workgroups of 64 rows per CU, and at four in a
-// causal grid, whose heaviest tile a large tile's time follows.  BH32 D128
-// S1000: causal 33 us on 256 rows, 19 on 64 (15 with BH8); not causal 33 and
-// 26; S2048: causal 61 and 49, not causal (four per CU) 67 and 86; BH128
-// S1024 causal (eight per CU) 50 and 56.  Above D 128 the large tile is 128
-// rows and the line at one workgroup per CU (BH8 S1000 causal 39 and 27).
-int64_t query_tile(int64_t tile, int64_t BH, int64_t Sq, int64_t D, bool causal, int cus) {
-  const int64_t per_cu = D > 128 ? 1 : causal ? 4 : 2;
-  return BH * cdiv64(Sq, 64) <= per_cu * cus ? 64 : tile;
-}
-
 template <bool H, bool KREG>
 void launch_attention(AttnParams p, int64_t D, int64_t tile_m, hipStream_t st) {
-  tile_m = query_tile(tile_m, p.BH, p.Sq, D, p.causal != 0, p.cus);
   p.nqt = (int)cdiv64(p.Sq, tile_m);
   const dim3 grid((unsigned)(p.BH * p.nqt)), b4(256), b8(512);
   auto launch = [&](auto kern, dim3 block) { hipLaunchKernelGGL(kern, grid, block, 0, st, p); };
@@ -610,7 +593,7 @@ int attention_impl(const void* k, const void* v, const void* q, void* out, int64
     return loom_fail(err, errlen, LOOM_EINVAL, "attention: causal needs Sq == Skv");
   // tile_m is bounded by Sq (natural_ub) and runs on the smallest built
   // query tile covering it (the largest above them: 256, or 128 for head dims
-  // above 128), or on 64 rows (query_tile)
+  // above 128)
   static const int64_t kQTiles[4] = {64, 128, 192, 256};
   const int64_t wm = loom_fit_tile(tile_m, Sq, kQTiles, D > 128 ? 2 : 4);
   if (wm == 0)

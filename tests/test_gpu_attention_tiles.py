@@ -1,6 +1,6 @@
-"""The attention kernels on both sides of the rule that picks the workgroup's
-query tile: grids large enough that a binding's own tile (128, 192, 256) runs,
-and small ones, which run as 64 rows whose keys two waves share.  Sampled heads
+"""The attention kernels on both sides of the rule that picks the query tile of
+a call that leaves it free (small grids: 64 rows whose keys two waves share),
+and bound tiles (64 .. 256), which run as bound on any grid.  Sampled heads
 against the CPU oracle, at attention's bar (tests/test_gpu_parity.py).
 """
 import math
@@ -52,7 +52,27 @@ def test_large_grids_run_the_bound_tile(lh, D, tile_m, Sq, Skv, causal):
     (64, 256, 72, 256, False), (2, 130, 33, 128, False), (2, 64, 32, 128, False),
     (2, 70, 31, 64, False), (1, 1, 1, 128, False), (2, 96, 96, 256, True)])
 def test_small_grids(lh, BH, Sq, Skv, D, causal):
-    _check(lh, BH, Sq, Skv, D, causal, min(256, Sq), range(0, BH, max(1, BH // 3)))
+    for tile_m in (None, min(256, Sq)):
+        _check(lh, BH, Sq, Skv, D, causal, tile_m, range(0, BH, max(1, BH // 3)))
+
+
+@pytest.mark.parametrize("D,tile_m", [(64, 128), (64, 192), (64, 256), (96, 128), (96, 192),
+                                      (96, 256), (128, 64), (128, 128), (128, 192), (128, 256),
+                                      (256, 64), (256, 128)])
+@pytest.mark.parametrize("Skv", [256, 61])
+def test_bound_tile_on_any_grid(lh, D, tile_m, Skv):
+    """A bound tile runs as bound whatever the grid: the heads of a small call
+    are bit for bit those of a large one, and tiles of more than 64 rows, which
+    sum a row's keys in one order, agree with each other."""
+    rng = np.random.default_rng(D + tile_m)
+    BH, Sq = 300, 256
+    k, v, q = (dev(rng_bf16(rng, s)) for s in ((BH, D, Skv), (BH, Skv, D), (BH, Sq, D)))
+    print(f"attention bound tile {tile_m} D{D} Skv{Skv}", flush=True)
+    large = lh.attention(k, v, q, tile_m=tile_m)
+    small = lh.attention(k[:2].contiguous(), v[:2].contiguous(), q[:2].contiguous(), tile_m=tile_m)
+    assert torch.equal(small, large[:2])
+    if tile_m > 64:
+        assert torch.equal(large, lh.attention(k, v, q, tile_m=128))
 
 
 @pytest.mark.parametrize("hidden", [(32, 64), (0, 32), (0, 64), (64, 128)])

@@ -109,6 +109,23 @@ def test_prologue_plans(base):
     assert accepted or base == f32
 
 
+# either side of each line: 64-row workgroups per CU of 256 (one above D 128,
+# two, four when causal), and short Sq
+@pytest.mark.parametrize("BH,Sq,D,causal,want", [
+    (8, 4096, 128, False, 64), (8, 4097, 128, False, 256), (16, 4096, 64, True, 64),
+    (16, 4097, 64, True, 256), (4, 4096, 256, True, 64), (4, 4097, 136, False, 128),
+    (1, 40, 64, False, 40), (1, 1000, 80, True, 64), (600, 40, 128, False, 40),
+    (600, 100, 128, False, 64), (600, 200, 128, False, 192), (600, 40, 128, True, 40)])
+def test_free_query_tile(BH, Sq, D, causal, want):
+    t = dict(tile_b=None, tile_m=None, tile_n=None)
+    dims = BH, Sq, Sq, D
+    assert lh._tiles("attention", dims, causal, **t)[1] == want
+    sig = (bf, (BH, D, Sq), bf, (BH, Sq, D), bf, (BH, Sq, D))
+    assert lh._plan("attention", sig, tuple(t.items()), causal)[3][1] == want
+    for tile in (16, min(128, Sq), Sq):      # a bound one stays
+        assert lh._tiles("attention", dims, causal, **{**t, "tile_m": tile})[1] == tile
+
+
 class _OnDevice(torch.Tensor):
     """A tensor without memory that says it lies on device 0, as _enter asks."""
 
