@@ -322,12 +322,23 @@ def _out_like(out, shape, e, dev):
 # on the host, of which the launch is 3.4, and takes 5.8; a decode step (two
 # launches, output and workspace allocated) 20.5 and 12.7.
 
+#: the tiles of a call that gives none, in the entry point's order
+_FREE = {f: tuple((s, None) for s in symbols.split()) for f, symbols in {
+    "matmul": "tile_m tile_n tile_k",
+    "batch_matmul": "tile_b tile_m tile_n tile_k",
+    "split_k_matmul_gather": "tile_m tile_n tile_k",
+    "attention": "tile_b tile_m tile_n",
+    "flash_decode": "tile_b tile_s tile_n",
+    "helion_mamba2_chunk_scan_kernel": "tile_b tile_h tile_c tile_m tile_n tile_k",
+}.items()}
+
+
 @functools.lru_cache(maxsize=1024)
 def _plan(func: str, sig: tuple, given: tuple, causal: bool = False):
     """(entry point, its name, extents, tiles, element type, output shape) of
     a signature: sig holds each input's dtype and shape, given the tiles as
-    (symbol, value) pairs, causal whether it is a causal attention.  None when
-    an input does not fit."""
+    (symbol, value) pairs (none of them: all free), causal whether it is a
+    causal attention.  None when an input does not fit."""
     dtypes, shapes = sig[0::2], [tuple(x) for x in sig[1::2]]
     try:
         dims = _dims_of_shapes(func, shapes)
@@ -339,7 +350,7 @@ def _plan(func: str, sig: tuple, given: tuple, causal: bool = False):
         for dt, sh, (_, kind, want) in zip(dtypes, shapes, spec):
             if sh != tuple(want) or dt != (e if kind == "e" else side):
                 return None
-        tiles = tuple(_tiles(func, dims, causal, **dict(given)))
+        tiles = tuple(_tiles(func, dims, causal, **dict(given or _FREE[func])))
     except (ValueError, TypeError, RuntimeError, KeyError):
         return None
     name = "loom_hip_" + func + ("_f16" if e == _f16 else "")
@@ -427,11 +438,12 @@ def matmul(x, y, out=None, *, tile_m=None, tile_n=None, tile_k=None):
     """@matmul (examples/mm/IR/00_from_helion_frontend.mlir:2): out = x . y.
     Tiles left as None take the preferred binding for the extents; with all
     three left so, a long K over few tiles is summed in slabs (_slabs)."""
-    go = _enter("matmul", (x, y), out,
+    free = tile_m is tile_n is tile_k is None
+    go = _enter("matmul", (x, y), out, () if free else
                 (("tile_m", tile_m), ("tile_n", tile_n), ("tile_k", tile_k)))
     if go:
         plan, out, st = go
-        if tile_m is None and tile_n is None and tile_k is None:
+        if free:
             tk = _slabs(*plan[2])
             if tk and _matmul_slabs(plan, x, y, out, tk, st):
                 return out
@@ -449,6 +461,7 @@ def matmul(x, y, out=None, *, tile_m=None, tile_n=None, tile_k=None):
 def batch_matmul(arg0, arg1, arg2=None, *, tile_b=None, tile_m=None, tile_n=None, tile_k=None):
     """@batch_matmul (examples/bmm_2Dmesh/IR/00_from_helion_frontend.mlir:4)."""
     go = _enter("batch_matmul", (arg0, arg1), arg2,
+                () if tile_b is tile_m is tile_n is tile_k is None else
                 (("tile_b", tile_b), ("tile_m", tile_m), ("tile_n", tile_n), ("tile_k", tile_k)))
     if go:
         plan, arg2, st = go
@@ -474,6 +487,7 @@ def split_k_matmul_gather(a, b, out=None, partials=None, *, tile_m=None, tile_n=
     Returns (out [M,N] bf16, partials [S,M,N] fp32 -- the gathered K-slab
 products, S = ceil(K / tile_k))."""
     go = _enter("split_k_matmul_gather", (a, b), out,
+                () if tile_m is tile_n is tile_k is None else
                 (("tile_m", tile_m), ("tile_n", tile_n), ("tile_k", tile_k)))
     if go:
         plan, o, st = go
@@ -510,6 +524,7 @@ def attention(k, v, q, out=None, *, scale=None, causal=False, tile_b=None, tile_
     ``scale`` defaults to 1/sqrt(D)."""
     causal = bool(causal)
     go = _enter("attention", (k, v, q), out,
+                () if tile_b is tile_m is tile_n is None else
                 (("tile_b", tile_b), ("tile_m", tile_m), ("tile_n", tile_n)), causal)
     if go:
         plan, out, st = go
@@ -556,6 +571,7 @@ def flash_decode(k, v, q, out=None, workspace=None, *, scale=None, tile_b=None, 
     k [B,D,S] (transposed), v [B,S,D], q [B,H,D] -> out [B,H,D].  With
     ``return_partials`` also returns the gathered (lse [ns,B,H], o [ns,B,H,D])."""
     go = _enter("flash_decode", (k, v, q), out,
+                () if tile_b is tile_s is tile_n is None else
                 (("tile_b", tile_b), ("tile_s", tile_s), ("tile_n", tile_n)))
     if go:
         plan, out, st = go
@@ -623,6 +639,7 @@ def helion_mamba2_chunk_scan_kernel(cb, x, dt, dA_cumsum, C, D, prev_states_T, o
     f16 call (x in f16): every tensor f16, the reference's own signature."""
     f = "helion_mamba2_chunk_scan_kernel"
     go = _enter(f, (cb, x, dt, dA_cumsum, C, D, prev_states_T), out,
+                () if tile_b is tile_h is tile_c is tile_m is tile_n is tile_k is None else
                 (("tile_b", tile_b), ("tile_h", tile_h), ("tile_c", tile_c), ("tile_m", tile_m),
                  ("tile_n", tile_n), ("tile_k", tile_k)))
     if go:

@@ -74,6 +74,8 @@ def test_plans_match_the_full_checks(func, base, tile):
         except (ValueError, TypeError, RuntimeError):
             want = None
         assert (plan is None) == (want is None), (func, shapes, types)
+        if tile is None:      # a call that gives no tile
+            assert lh._plan(func, sig, ()) == plan
         if plan:
             accepted += 1
             assert plan[2:] == want
