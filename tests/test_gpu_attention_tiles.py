@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from oracle import from_bf16, to_bf16
+from oracle import from_bf16, from_f16, to_bf16, to_f16
 from tests.conftest import assert_close
 from tests.test_gpu_parity import ATTN_TOL, dev, host, rng_bf16
 
@@ -26,13 +26,20 @@ def lh():
 
 
 def _check(lh, BH, Sq, Skv, D, causal, tile_m, heads):
-    rng = np.random.default_rng(BH + 7 * Sq + Skv + D)
-    k, v, q = rng_bf16(rng, (BH, D, Skv)), rng_bf16(rng, (BH, Skv, D)), rng_bf16(rng, (BH, Sq, D))
-    print(f"attention tile BH{BH} Sq{Sq} Skv{Skv} D{D} causal={causal} tile {tile_m}", flush=True)
-    got = from_bf16(host(lh.attention(dev(k), dev(v), dev(q), causal=causal, tile_m=tile_m)))
+    """In bf16 and in f16: each type has its own build of every tile."""
     h = list(heads)
-    ref = from_bf16(oracle.attention(k[h], v[h], q[h], 1 / math.sqrt(D), causal, 1, 64, 64))
-    assert_close(got[h], ref, **ATTN_TOL, what=f"tile {tile_m} BH{BH} Sq{Sq} Skv{Skv} D{D} {causal}")
+    for name, to, back, dtype in (("bf16", to_bf16, from_bf16, torch.bfloat16),
+                                  ("f16", to_f16, from_f16, torch.float16)):
+        rng = np.random.default_rng(BH + 7 * Sq + Skv + D)
+        k, v, q = (to(rng.standard_normal(s, dtype=np.float32))
+                   for s in ((BH, D, Skv), (BH, Skv, D), (BH, Sq, D)))
+        what = f"{name} tile {tile_m} BH{BH} Sq{Sq} Skv{Skv} D{D} {causal}"
+        print("attention", what, flush=True)
+        got = lh.attention(*(dev(t).view(dtype) for t in (k, v, q)), causal=causal, tile_m=tile_m)
+        assert got.dtype == dtype
+        with oracle.element_type(name):
+            ref = back(oracle.attention(k[h], v[h], q[h], 1 / math.sqrt(D), causal, 1, 64, 64))
+        assert_close(back(host(got))[h], ref, **ATTN_TOL, what=what)
 
 
 # more than four workgroups of 64 rows per CU of 256
