@@ -2,8 +2,9 @@
 
 Every kernel forms its per-batch, per-head and per-chunk bases in 64-bit
 arithmetic and keeps per-lane offsets within one tile, row block or head;
-the GEMM kernels whose LDS-DMA copies take 32-bit per-lane offsets run only
-when a tile's rows fit them (leading dimensions below 2^22), larger ones
+the GEMM kernels whose copies take 32-bit per-lane offsets run only when a
+tile's rows fit them (the pipelined kernels up to 2^23, 2^24 and 2^25 columns
+at tiles of 256, 128 and 64 rows, the ragged one up to 2^22), larger ones
 take the 64-bit fallback kernels.  Each case here puts at least one operand,
 output or workspace past 2^32 bytes and checks the elements that live past
 that boundary (the last batch, head, rows or columns; for the GEMMs also
@@ -74,7 +75,7 @@ def _announce(what):
     ("x past 4 GiB", 69632, 256, 32768),
     ("y past 4 GiB", 256, 69632, 32768),
     ("out past 4 GiB", 47104, 47104, 256),
-    ("out past 4 GiB, K 64 (fallback kernels)", 47104, 47104, 64)])
+    ("out past 4 GiB, K 64 (half a round of stages)", 47104, 47104, 64)])
 def test_matmul_past_4gib(lh, case, M, N, K):
     x, y = _ints((M, K), 1), _ints((K, N), 2)
     out = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
@@ -117,7 +118,7 @@ def test_batch_matmul_past_4gib(lh, case, Bt, M, N, K):
 
 @pytest.mark.parametrize("case,M,N,K,tile_k,tiles", [
     ("partials past 4 GiB", 8192, 8192, 17408, 1024, (256,)),
-    ("A and B rows past 2^22 elements (fallback kernels)", 512, 512, 5242880, 16384, (256, 128))])
+    ("A rows at offsets past 2^31 bytes in a tile", 512, 512, 5242880, 16384, (256, 128))])
 def test_split_k_past_4gib(lh, case, M, N, K, tile_k, tiles):
     a, b = _ints((M, K), 5), _ints((K, N), 6)
     S = -(-K // tile_k)
@@ -135,6 +136,18 @@ def test_split_k_past_4gib(lh, case, M, N, K, tile_k, tiles):
                                       err_msg=f"split_k {case} partials, tile {t}")
         np.testing.assert_array_equal(host(out[rs, cs].contiguous()), ref,
                                       err_msg=f"split_k {case} output, tile {t}")
+
+
+@pytest.mark.parametrize("case,M,N,K", [
+    ("rows of A past the pipelined kernels' offsets (fallback kernel)", 65, 16, (1 << 25) + 64),
+    ("rows of A past the ragged kernel's offsets (fallback kernel)", 513, 16, (1 << 22) + 1)])
+def test_matmul_rows_past_32_bit_offsets(lh, case, M, N, K):
+    x, y = _ints((M, K), 13), _ints((K, N), 14)
+    assert _big(x)
+    _announce(f"matmul {case} M{M} N{N} K{K}")
+    got = host(lh.matmul(x, y, tile_m=64, tile_n=16, tile_k=64))
+    rows = [0, 31, M - 2, M - 1]
+    np.testing.assert_array_equal(got[rows], oracle.matmul(host(x[rows]), host(y)), err_msg=case)
 
 
 # --------------------------------------------------------------- attention
