@@ -526,7 +526,7 @@ int build_scope(const std::string& f, const int64_t* d, int nd, Scope& sc, std::
   // the reference's 32-alignment of inner tile dimensions
   // (hw_alignment.cpp:16).  It runs on the smallest built workgroup tile
   // covering it, or the largest built one above them all (loom_fit_tile in
-  // csrc/common.h); no kernel's result depends on that choice.
+  // csrc/common.h); no kernel's result depends on that choice beyond rounding.
   auto ub = [&](const char* sym, long long extent) { sc.hard.push_back(jrange(sym, 1, extent)); };
   auto tiled = [&](const char* sym, long long extent) {
     ub(sym, extent);

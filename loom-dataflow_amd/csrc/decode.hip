@@ -14,10 +14,11 @@
 // more arithmetic than the fp32 VALU peak, so S^T = K^T . Q^T and
 // O^T += V^T . P^T run on MFMA and the kernel stays bound by the stream.
 // One workgroup (4 waves) per (batch, split, group of 32 query heads):
-//   - decode_dma_kernel (S a multiple of 8, or any S above D 128 or 32
-//     heads or in splits up to 512 keys, with K staged through registers; 4 waves for up to 32 heads, 8
-//     for 64): K and V stream through a ring of LDS-DMA stages (four, two at
-//     D 256) and reach the MFMAs by transposed LDS reads (described at the
+//   - decode_dma_kernel (S a multiple of 8, or any S above D 128 or 32 heads or
+//     in splits up to 512 keys, with K staged through registers; 4 waves for
+//     up to 32 heads, 8 for 64): K and V stream through a ring of LDS-DMA
+//     stages (three; two at D 256 and in grids of more than one workgroup per
+//     CU) and reach the MFMAs by transposed LDS reads (described at the
 //     kernel);
 //   - decode_split_kernel (other S, up to 32 heads and D 128, splits above 512
 //     keys): raw buffer loads straight into

@@ -937,16 +937,18 @@ bool launch_persist(GemmParams p, bool out_f32, hipStream_t st) {
 // would pass column N is loaded ending there and shifted down; its columns
 // past N are never stored.  Needs ke >= 8 and N >= 8.
 //
-// Bound: the loads' issue.  A 16-byte load at an odd element costs about four
-// times one on a dword (T 64, 2048^3: 36 us with every row on a dword, 67 us
-// with every row off one), and half of an odd extent's rows start at one; then
+// Bound: the loads' address path.  A wave's 16-byte load costs it 65 cycles
+// with every row at an odd element, 21 with every row on a dword, and 41 where
+// they alternate, as the rows of an odd leading dimension do: the mean, so
+// loads of rows of one kind would save nothing (T 64, 2048^3: 36 us with every
+// row on a dword, 67 us with every row off one); then
 // the step's chain of LDS store, barrier, LDS read and MFMA, which two or three
 // workgroups per CU overlap.  Against the element-load kernel (eight 2-byte
 // loads a piece) that ran these shapes before, M 1003 N 1531 K 2051: 214 ->
 // 26 us (242 TFLOP/s).  Four stages of loads in flight instead of two took the
 // same time and 64 more VGPRs; the odd pieces as an aligned 16-byte load, the
-// next dword and a byte shift: 27 against 35 us on the 64 tile (every row odd,
-// 1024x1536x2048) but 47 against 35 on the 128 tile.
+// next dword and a byte shift: 25 to 27 against 35 us on the 64 tile (every row
+// odd, 1024x1536x2048) but 39 to 47 against 35 on the 128 tile.
 // ---------------------------------------------------------------------------
 typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));   // 16 bytes at any element
 
@@ -1351,8 +1353,9 @@ int matmul_impl(const void* x, const void* y, void* out, int64_t M, int64_t N, i
   p.k_slab = K;
   p.split = 0;
   p.nz = 1;
-  // the vector-store kernels also need a 16-byte-aligned C; others take the
-  // register-staged kernel (element stores)
+  // the LDS-DMA kernels need 16-byte rows of A, B and C; others take the ragged
+  // kernel (16-byte accesses at any element), and where its conditions fail
+  // (K or N below 8, leading dimensions of 2^22 or more) the register-staged one
   const bool al = K % 8 == 0 && N % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(out);
   if (loom_validate_only()) return loom_ok(err, errlen);
   return loom_launched(launch_gemm<H>(p, wg, al, false, static_cast<hipStream_t>(stream)), err,

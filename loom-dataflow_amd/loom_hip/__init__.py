@@ -485,7 +485,7 @@ def split_k_matmul_gather(a, b, out=None, partials=None, *, tile_m=None, tile_n=
     """@split_k_matmul_gather (examples/split_k_mm_gather/IR/00_from_helion_frontend.mlir:2).
 
     Returns (out [M,N] bf16, partials [S,M,N] fp32 -- the gathered K-slab
-products, S = ceil(K / tile_k))."""
+    products, S = ceil(K / tile_k))."""
     go = _enter("split_k_matmul_gather", (a, b), out,
                 () if tile_m is tile_n is tile_k is None else
                 (("tile_m", tile_m), ("tile_n", tile_n), ("tile_k", tile_k)))
