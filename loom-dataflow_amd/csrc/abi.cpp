@@ -851,7 +851,7 @@ int loom_hip_preferred_block_sizes(const char* func, const int64_t* dims, int nd
     // against 50).  Above D 128 the large tile is 128 rows and the line at one
     // workgroup per CU (BH8 S1000 causal 27 against 39).
     const long long top = d[3] > 128 ? 128 : 256;
-    if (d[0] * ceil_div(d[1], 64) <= (d[3] > 128 ? 1 : 2) * kCUs)
+    if (ceil_div(d[1], 64) <= (d[3] > 128 ? 1 : 2) * kCUs / d[0])   // no product that overflows
       b["tile_m"] = bound(64, d[1]);
     else
       b["tile_m"] = d[1] >= top ? top : d[1] >= 192 ? 192 : d[1] >= 128 ? 128 : bound(64, d[1]);

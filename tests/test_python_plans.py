@@ -117,7 +117,8 @@ def test_prologue_plans(base):
     (8, 4096, 128, False, 64), (8, 4097, 128, False, 256), (16, 4096, 64, True, 64),
     (16, 4097, 64, True, 256), (4, 4096, 256, True, 64), (4, 4097, 136, False, 128),
     (1, 40, 64, False, 40), (1, 1000, 80, True, 64), (600, 40, 128, False, 40),
-    (600, 100, 128, False, 64), (600, 200, 128, False, 192), (600, 40, 128, True, 40)])
+    (600, 100, 128, False, 64), (600, 200, 128, False, 192), (600, 40, 128, True, 40),
+    (171, 192, 64, False, 192), (170, 192, 64, False, 64), (1 << 40, 1 << 40, 128, False, 256)])
 def test_free_query_tile(BH, Sq, D, causal, want):
     t = dict(tile_b=None, tile_m=None, tile_n=None)
     dims = BH, Sq, Sq, D
